@@ -281,7 +281,10 @@ def run(state):
     if kind == "batch":
         b = state["batch"]
         b.run(case["steps"])
-        return [b.macros(c) for c in range(case["cases"])]
+        fields = [b.macros(c) for c in range(case["cases"])]
+        if case["storage"] == "f32s":  # the program keeps what FP32 populations determine
+            fields = [tuple(a.astype(np.float32) for a in f) for f in fields]
+        return fields
     if kind == "adjoint":
         rho0, ux0, uy0, uxt, uyt = state["fields"]
         loss = state["eng"].forward(rho0, ux0, uy0, 1.0 / case["tau"], uxt, uyt)
