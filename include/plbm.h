@@ -272,10 +272,11 @@ double plbm_magic_number(double le, double ld);
 int plbm_set_launch(plbm_lattice *h, int model, int block, int xcd_remap);
 int plbm_get_launch(const plbm_lattice *h, int model, int *block, int *xcd_remap);
 /* Temporal blocking of plbm_run: steps advanced per pass over HBM (1 = the single-step
- * kernel; 2..8 = that many fused steps per launch, each wavefront walking a segment of
- * columns with the intermediate states in registers; 0 = chosen from the grid size: 8
- * when the default work split gives at least 512 wavefronts, about 512^2 and larger,
- * else 1).  In F64 storage the results are bit-identical for every setting;
+ * kernel; 2..8 = that many fused steps per launch, in tiles held in LDS on small and medium
+ * grids and by wavefronts walking segments of columns on larger ones; 0 = chosen from the
+ * grid size: launches of up to 8 steps, or single steps on wide, flat grids beyond the
+ * tiles' limit, and while the lattice's stream is being captured on grids below about
+ * 512^2).  In F64 storage the results are bit-identical for every setting;
  * the shifted storages agree to roundoff (their collisions allow FMA contraction, which
  * the compiler places per kernel).  plbm_run keeps the reference's slot contents (latest
  * in *iold, the state one step earlier in *inew); with passes of more than one step it

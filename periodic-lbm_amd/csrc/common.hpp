@@ -122,6 +122,8 @@ struct StepArgs {
     // Pass kernels only: when non-null, the pass also stores the state one step before
     // its last (level NS-1, post-collision) here, in the layout of dst.
     void *lag = nullptr;
+    // Tile passes in FP16 storage: round every level to the storage, as single steps do.
+    int round_levels = 0;
 };
 
 // Strip length (columns per thread) of the stencil kernels that walk along x with a
@@ -204,10 +206,18 @@ inline int plane_from_host(double *dev, const double *host, size_t ld, size_t ny
 struct plbm_lattice;
 
 namespace plbm {
-// One temporally blocked pass of ns (2..8) steps src -> dst; with lag non-null it also
-// stores the state one step before the pass's last there (multistep.hip).
+// One temporally blocked pass of ns (2..8) steps src -> dst, in LDS tiles (tile.hip) or by
+// column walks (multistep.hip), whichever suits the grid; with lag non-null it also stores
+// the state one step before the pass's last there.
 int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
-                 void *lag = nullptr);
+                 void *lag = nullptr, bool round_levels = false);
+// Tile passes (tile.hip): whether the lattice's passes run in tiles, and one such pass
+// (round_levels: FP16 storage rounds every level, as single steps do).
+bool tile_grid(const plbm_lattice *h, int model);
+bool tile_cells(int storage, int model, long long cells);
+int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
+                bool round_levels);
+double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
 // Run bookkeeping shared by the pass runs (multistep.hip): pass depths of a run, the
 // lattice's third buffer (nullptr when it cannot be allocated), and the final assignment
 // of device storage to slots.

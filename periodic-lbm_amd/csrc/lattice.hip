@@ -382,9 +382,8 @@ int launch_step_cfg(plbm_lattice *h, int model, const void *src, void *dst, Laun
     });
 }
 
-int run_steps(plbm_lattice *h, int model, int ns, int lag_ns, int nsteps, int *iold,
-              int *inew);
-int default_steps_per_launch(const plbm_lattice *h);
+int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew);
+int default_steps_per_launch(const plbm_lattice *h, int model);
 
 int launch_step(plbm_lattice *h, int model, const void *src, void *dst) {
     PLBM_REQUIRE(model >= PLBM_BGK && model <= PLBM_BGK_SPLIT, PLBM_ERR_ARG,
@@ -765,8 +764,7 @@ int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) try {
     PLBM_TRY(check_buf(h, *inew));
     PLBM_REQUIRE(*iold != *inew, PLBM_ERR_ARG, "iold == inew");
     PLBM_TRY(require_params(h));
-    const int ns = h->cfg[model].ns > 0 ? h->cfg[model].ns : default_steps_per_launch(h);
-    return run_steps(h, model, ns, h->cfg[model].lag_ns, nsteps, iold, inew);
+    return run_steps(h, model, nsteps, iold, inew);
 } catch (...) {
     return plbm::host_exception();
 }
@@ -930,7 +928,7 @@ int plbm_set_steps_per_launch(plbm_lattice *h, int model, int ns) try {
 int plbm_get_steps_per_launch(const plbm_lattice *h, int model, int *ns) try {
     PLBM_REQUIRE(h && ns, PLBM_ERR_ARG, "null argument");
     PLBM_REQUIRE(model >= PLBM_BGK && model <= PLBM_BGK_SPLIT, PLBM_ERR_ARG, "unknown collision model");
-    *ns = h->cfg[model].ns > 0 ? h->cfg[model].ns : default_steps_per_launch(h);
+    *ns = h->cfg[model].ns > 0 ? h->cfg[model].ns : default_steps_per_launch(h, model);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();

@@ -85,8 +85,23 @@ int max_steps_per_pass(int) { return kMaxPassSteps; }
 // each wavefront's sequential walk.
 int default_pass_segments(int nx) { return std::max(1, std::min(64, nx / 8)); }
 
+// Whether the default work split gives the column walk at least 512 wavefronts.
+static bool enough_walks(const plbm_lattice *h) {
+    const int vr = multi_rows(storage_bytes(h->storage), kMaxPassSteps);
+    return (long)((h->ny + vr - 1) / vr) * default_pass_segments(h->nx) >= 512;
+}
+
+// Most steps of a launch of plbm_run when the caller has not chosen: 8 where it runs in
+// tiles, or where the column walk has at least 512 wavefronts; else single steps (wide and
+// flat grids beyond the tiles' limit).
+int default_steps_per_launch(const plbm_lattice *h, int model) {
+    return enough_walks(h) || tile_grid(h, model) ? kMaxPassSteps : 1;
+}
+
 int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
-                 void *lag) {
+                 void *lag, bool round_levels) {
+    if (ns >= 2 && ns <= kMaxPassSteps && tile_grid(h, model))
+        return launch_tile(h, model, ns, src, dst, lag, round_levels);
     StepArgs a{};
     a.src = src;
     a.dst = dst;
@@ -227,8 +242,31 @@ static int timing_mark(plbm_lattice *h, int depth) {
     return PLBM_OK;
 }
 
-int run_steps(plbm_lattice *h, int model, int ns, int lag_ns, int nsteps, int *iold,
-              int *inew) {
+//
+// A grid that takes tiles chooses the depth itself when the caller has not
+// (plbm_set_steps_per_launch): the cheapest of 2..8 (pick_tile), spread evenly over the
+// passes.  FP16 storage rounds a state whenever it is stored, so there the depth shows in
+// the results: where single steps were the automatic choice before (grids of fewer than 512
+// column walks) every level is rounded as they round it, elsewhere the depth stays 8.
+// While the stream is being captured, such small grids keep single steps: their slots do not
+// move, so that a caller's graph can be replayed.
+int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
+    int ns = h->cfg[model].ns, lag_ns = h->cfg[model].lag_ns;
+    bool even = false, round_levels = false;
+    if (ns == 0) {
+        const bool walks = enough_walks(h);
+        ns = walks ? kMaxPassSteps : 1;
+        if (tile_grid(h, model) && (!walks || h->storage != PLBM_F16S)) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (!walks) PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
+            if (cap == hipStreamCaptureStatusNone) {
+                int shape;
+                pick_tile(h->nx, h->ny, 2, kMaxPassSteps, &shape, &ns);
+                even = true;
+                round_levels = h->storage == PLBM_F16S;
+            }
+        }
+    }
     h->run_depths.clear();
     PLBM_TRY(timing_mark(h, 0));
     if (ns <= 1 || nsteps < 2) {
@@ -244,7 +282,7 @@ int run_steps(plbm_lattice *h, int model, int ns, int lag_ns, int nsteps, int *i
     void *aux = pass_aux(h);
     auto launch = [&](int k, void *lag) {
         PLBM_TRY(k == 1 ? launch_step(h, model, latest, other)
-                        : launch_multi(h, model, k, latest, other, lag));
+                        : launch_multi(h, model, k, latest, other, lag, round_levels));
         return timing_mark(h, k);
     };
     if (aux == nullptr) {
@@ -256,7 +294,8 @@ int run_steps(plbm_lattice *h, int model, int ns, int lag_ns, int nsteps, int *i
         finish_run(h, a0, b0, nsteps, other, latest, nullptr, iold, inew);
         return PLBM_OK;
     }
-    const std::vector<int> plan = lag_pass_plan(nsteps, ns, lag_ns);
+    const std::vector<int> plan =
+        even ? pass_plan(nsteps, ns) : lag_pass_plan(nsteps, ns, lag_ns);
     for (size_t p = 0; p + 1 < plan.size(); ++p) {
         PLBM_TRY(launch(plan[p], nullptr));
         std::swap(latest, other);
@@ -264,21 +303,6 @@ int run_steps(plbm_lattice *h, int model, int ns, int lag_ns, int nsteps, int *i
     PLBM_TRY(launch(plan.back(), aux));
     finish_run(h, a0, b0, nsteps, other, aux, latest, iold, inew);
     return PLBM_OK;
-}
-
-}  // namespace plbm
-
-namespace plbm {
-
-// Steps per pass when the caller has not chosen: 8 where the default work split gives at
-// least 512 wavefronts, else single steps.  TRT, 8 steps per pass against single steps,
-// GLUPS (FP64): 512^2 52.6 / 31.9, 1024^2 101.5 / 35.4, 2048^2 153.6 / 40.8, 4096^2 187
-// / 42.5; 320^2 (35 wavefronts of 64 columns) 36 against 5 us per step.  At 8192^2 8 is
-// the fastest depth for every storage.
-int default_steps_per_launch(const plbm_lattice *h) {
-    const int vr = multi_rows(storage_bytes(h->storage), kMaxPassSteps);
-    const long waves = (long)((h->ny + vr - 1) / vr) * default_pass_segments(h->nx);
-    return waves >= 512 ? kMaxPassSteps : 1;
 }
 
 }  // namespace plbm

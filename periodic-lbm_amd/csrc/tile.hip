@@ -1,0 +1,115 @@
+// tile.hip — temporally blocked passes of small and medium grids, held in LDS.
+//
+// The column walk of multistep.hip needs a long walk per wavefront and about a thousand
+// wavefronts: below about 1000^2 its start-up columns (2 NS per segment) and idle SIMDs cost
+// more than the steps, and below about 500^2 single steps, one launch of 2.5-3.5 us each,
+// were faster.  Here a workgroup advances one rectangular tile ns steps in LDS (tile.hpp):
+// level 1 is pulled from global memory over the tile and its halo of ns - 1 cells on each
+// side, each further level is one cell smaller on every side, and the last is stored.  What
+// bounds it: a CU's VALU issue plus the LDS traffic that does not overlap it (512^2 TRT FP64,
+// 8 steps: 58% of the issue slots of the busy CUs, 38% LDS active, a fifth of that bank
+// conflicts where a wavefront crosses a column), the launch for the smallest grids.  Two
+// cells per thread and iteration, to overlap one's LDS reads with the other's collision,
+// measured 3-20% slower.
+//
+// us per step, single steps / column walk of 8 / tiles: 64^2 BGK FP64 3.4 / 5.5 / 1.1;
+// 192^2 TRT FP64 3.6 / 4.9 / 1.2; 512^2 TRT FP64 8.3 / 5.0 / 2.3, FP32 4.3 / 3.5 / 1.6;
+// 1001 x 777 RR FP64 23.8 / 24.5 / 10.1; 1024^2 TRT FP64 29 / 10.0 / 8.4, FP32 16.4 / 5.8 /
+// 4.2.
+//
+// Per-cell arithmetic is collide_cell, as everywhere: FP64 results equal single steps bit
+// for bit, and the shifted FP64 / FP32 storages did on every case compared.
+#include "tile.hpp"
+
+namespace plbm {
+
+template <int MODEL, int ST, class SHAPE>
+__global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4)))
+    k_tile(StepArgs a, int ns, int nbx, int nby) {
+    const int b = xcd_remap(blockIdx.x, gridDim.x);  // neighbouring tiles share an L2
+    const int by = b % nby, bx = b / nby;
+    const int x0 = part_start(a.nx, nbx, bx), x1 = part_start(a.nx, nbx, bx + 1);
+    const int y0 = part_start(a.ny, nby, by), y1 = part_start(a.ny, nby, by + 1);
+    tile_steps<MODEL, ST, SHAPE>(a, ns, x0, x1 - x0, y0, y1 - y0);
+}
+
+double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
+    double best = 1e300;
+    for (int n = ns_min; n <= ns_max; ++n)
+        for (int s = 0; s < kTileShapes; ++s) {
+            int w, h;
+            tile_limits(s, n, &w, &h);
+            const long long nbx = (nx + w - 1) / w, nby = (ny + h - 1) / h;
+            w = (int)((nx + nbx - 1) / nbx);
+            h = (int)((ny + nby - 1) / nby);
+            const double per_cu = double((nbx * nby + kComputeUnits - 1) / kComputeUnits);
+            const double c = (kTileLaunchWork + per_cu * tile_work(s, n, w, h)) / n;
+            if (c < best) {
+                best = c;
+                *shape = s;
+                *ns = n;
+            }
+        }
+    return best;
+}
+
+// Grids up to this many cells take tiles: about where the column walk catches up.  us per
+// step at both sides' automatic depths, column walk / tiles, FP64 | FP32 | FP16:
+//   BGK  1200^2 19.4/14.6 | 8.7/6.9 | 8.5/7.2;  1400^2 21.6/22.3 | 10.3/8.8 | 10.0/9.5;
+//        2048^2 41.7/44.1 | 22.0/21.9 | 21.8/18.6;  3000 x 1500 - | - | 17.2/19.6;
+//        3000^2 73.0/92.1 | 36.4/47.9 | 33.9/38.9
+//   TRT  1000^2 10.5/10.3 | 6.4/5.9 | 6.3/4.5;  1200^2 11.7/13.1 | 7.3/6.4 | 7.1/6.4;
+//        1600^2 21.2/32.6 | 11.1/12.6 | 11.1/10.0;  2048^2 26.1/40.8 | 14.9/20.9 | 13.8/15.7
+//   RR   1200^2 27.8/17.5 | 12.4/9.3 | 12.2/9.9;  2048^2 62.5/55.2 | 31.7/26.3 | 30.7/25.6;
+//        2600^2 98.0/84.8 | 43.4/43.0 | 42.4/39.8;  3000^2 110.9/114.2 | 50.8/57.7 | 48.5/53.0
+bool tile_cells(int storage, int model, long long cells) {
+    const int bytes = (int)storage_bytes(storage);
+    const auto pick = [&](long long f64, long long f32, long long f16) {
+        return cells <= (bytes == 8 ? f64 : bytes == 4 ? f32 : f16);
+    };
+    if (model == PLBM_TRT) return pick(1050000, 2000000, 2000000);
+    if (model == PLBM_RR) return pick(7000000, 7000000, 4200000);
+    return pick(1800000, 4000000, 4200000);
+}
+
+// A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.
+bool tile_grid(const plbm_lattice *h, int model) {
+    return h->pass_segs == 0 && tile_cells(h->storage, model, (long long)h->nx * h->ny);
+}
+
+int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
+                bool round_levels) {
+    StepArgs a{};
+    a.src = src;
+    a.dst = dst;
+    a.lag = lag;
+    a.nx = h->nx;
+    a.ny = h->ny;
+    a.ldd = h->ldd;
+    a.cs = (size_t)9 * h->ldd;
+    a.omega = h->omega;
+    a.lambda_odd = h->lambda_odd;
+    a.omega_f = float(h->omega);
+    a.lambda_odd_f = float(h->lambda_odd);
+    a.scale = float(h->scale);
+    a.inv_scale = float(1.0 / h->scale);
+    a.round_levels = round_levels;
+    int shape = 0, wx, wy;
+    pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
+    tile_limits(shape, ns, &wx, &wy);
+    const int nbx = (h->nx + wx - 1) / wx, nby = (h->ny + wy - 1) / wy;
+    return dispatch_model(model, [&](auto M) {
+        return dispatch_storage(h->storage, [&](auto S) {
+            return dispatch_tile_shape(shape, [&](auto sh) {
+                using SH = decltype(sh);
+                hipLaunchKernelGGL((k_tile<decltype(M)::value, decltype(S)::value, SH>),
+                                   dim3((unsigned)(nbx * nby)), dim3(SH::T), 0, h->stream, a, ns,
+                                   nbx, nby);
+                PLBM_HIP(hipGetLastError());
+                return PLBM_OK;
+            });
+        });
+    });
+}
+
+}  // namespace plbm

@@ -1,0 +1,196 @@
+// tile.hpp — one workgroup's share of a temporally blocked pass held in LDS: NS fused
+// stream + collide steps of one rectangular tile (grids too small for the column walk of
+// multistep.hpp to fill the chip), shared by the single-lattice pass kernel (tile.hip) and
+// the batched engine (batch.hip).  See tile.hip for the scheme.
+#pragma once
+
+#include "common.hpp"
+#include "d2q9.hpp"
+#include "stepper.hpp"
+
+namespace plbm {
+
+// A tile's region at level 1 holds at most XW columns of H rows; T threads work on it.
+// LDS of the three shapes in FP64: 41, 78 and 159 of a CU's 160 KB, so that 3, 2 and 1
+// workgroups share a CU (16-24 wavefronts either way).  Measured and not kept: S with 256
+// threads (5-15% slower), M with 1024, L with 512 or 768 (3-13% slower), 18 x 18 (slower
+// beyond 64^2), 40 x 36, and 70 x 64 for 4-byte values (5-45% slower than L).
+template <int XW_, int H_, int T_, int MEM_>
+struct TileShape {
+    static constexpr int XW = XW_, H = H_, T = T_;
+    // cost of moving one cell between memory and LDS, in tenths of a cell's step: the
+    // more workgroups share a CU, the more of it overlaps another's steps
+    static constexpr int MEM = MEM_;
+};
+using TileS = TileShape<24, 24, 512, 7>;
+using TileM = TileShape<34, 32, 512, 8>;
+using TileL = TileShape<48, 46, 1024, 14>;
+constexpr int kTileShapes = 3;
+
+template <class F>
+inline int dispatch_tile_shape(int shape, F &&f) {
+    switch (shape) {
+    case 0: return f(TileS{});
+    case 1: return f(TileM{});
+    default: return f(TileL{});
+    }
+}
+
+// Most cells a tile of `shape` advances by ns steps: columns, rows.
+inline void tile_limits(int shape, int ns, int *w, int *h) {
+    dispatch_tile_shape(shape, [&](auto s) {
+        using S = decltype(s);
+        *w = S::XW - 2 * (ns - 1);
+        *h = S::H - 2 * (ns - 1);
+        return 0;
+    });
+}
+
+// Work of one tile of w x h cells and ns steps, in steps of a cell: the steps of its
+// shrinking levels, and the load of its region and the store of its cells.
+inline double tile_work(int shape, int ns, int w, int h) {
+    double c = 0;
+    for (int k = 0; k < ns; ++k) c += double(w + 2 * k) * (h + 2 * k);
+    dispatch_tile_shape(shape, [&](auto s) {
+        c += 0.1 * decltype(s)::MEM * (double(w + 2 * ns) * (h + 2 * ns) + double(w) * h);
+        return 0;
+    });
+    return c;
+}
+constexpr double kTileLaunchWork = 2500;  // a launch and its ramp, in the same unit
+constexpr int kComputeUnits = 256;        // MI355X
+
+// The shape and depth (in [ns_min, ns_max]) that cost the least per step on an nx x ny
+// grid; returns the cost of a step.  The busiest CU sets the time: ceil(tiles / 256) tiles
+// of the work above (TRT FP64: 0.9 ns a unit).  Over 32^2 to 2048^2, four collisions and
+// three storages the choice is within 8% of the fastest measured shape and depth.
+double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
+
+// Column / row boundary j of n cells cut into m nearly equal parts.
+__host__ __device__ inline int part_start(int n, int m, int j) {
+    return (int)((long long)n * j / m);
+}
+
+__host__ __device__ constexpr int opposite(int q) {
+    return q == 0 ? 0 : (q < 5 ? (q + 1) % 4 + 1 : (q - 3) % 4 + 5);
+}
+static_assert(opposite(1) == 3 && opposite(2) == 4 && opposite(3) == 1 && opposite(4) == 2 &&
+                  opposite(5) == 7 && opposite(6) == 8 && opposite(7) == 5 && opposite(8) == 6,
+              "opposite directions");
+
+__device__ __forceinline__ int wrap_index(int v, int n) {
+    if (v < 0 || v >= n) {
+        v %= n;
+        if (v < 0) v += n;
+    }
+    return v;
+}
+
+// The calling workgroup (SHAPE::T threads) advances cells [x0, x0 + w) x [y0, y0 + h) of
+// the grid described by `a` ns >= 2 steps, a.src -> a.dst, and, when a.lag is set, stores
+// the state one step before there.  w + 2 (ns - 1) <= XW, h + 2 (ns - 1) <= H.
+//
+// LDS holds one copy of the region's populations, updated in place.  A step pulls f_q(x)
+// from cell x - c_q, so writing the result where it was read from (A: the value of the
+// opposite direction goes to (x - c_q, q), where the next step's pull would send it) makes
+// the step after it a purely local one (B: direction p is read from (x, opposite(p)) and
+// written back to (x, p)).  Every LDS word is read and written by the same thread in a
+// step, so that one barrier per step suffices, any number of cells per thread works, and
+// half the LDS of a ping-pong pair holds the tile.
+template <int MODEL, int ST, class SHAPE>
+__device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, int w, int y0,
+                                           int h) {
+    using T = typename Traits<ST>::T;
+    using R = typename Traits<ST>::R;
+    constexpr int H = SHAPE::H, NT = SHAPE::T;
+    __shared__ R mem[SHAPE::XW * 9 * H];  // (lx, q, ly)
+    const T *__restrict__ s = static_cast<const T *>(a.src);
+    T *__restrict__ d = static_cast<T *>(a.dst);
+    T *__restrict__ lag = static_cast<T *>(a.lag);
+    const int nx = a.nx, ny = a.ny, halo = ns - 1;
+    const size_t L = (size_t)a.ldd;
+    // FP16 storage with a.round_levels: every level rounded as a single step's store and the
+    // next one's load round it
+    auto settle = [&](R(&f)[9]) __attribute__((always_inline)) {
+        if constexpr (ST == PLBM_F16S) {
+            if (a.round_levels)
+#pragma unroll
+                for (int q = 0; q < 9; ++q) f[q] = R(T(f[q] * a.scale)) * a.inv_scale;
+        }
+    };
+    auto store = [&](T *to, int lx, int ly, const R(&f)[9]) __attribute__((always_inline)) {
+        const int ox = lx - halo, oy = ly - halo;
+        if (ox < 0 || ox >= w || oy < 0 || oy >= h) return;
+        T *p = to + (size_t)(x0 + ox) * a.cs + (y0 + oy);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) store_pop<ST, false>(p + q * L, f[q], a.scale);
+    };
+
+    // level 1 from global memory, over the whole region
+    {
+        const int w1 = w + 2 * halo, h1 = h + 2 * halo, n = w1 * h1;
+        const float rh = 1.0f / float(h1);
+        for (int i = threadIdx.x; i < n; i += NT) {
+            const int lx = int((float(i) + 0.5f) * rh), ly = i - lx * h1;
+            const int x = wrap_index(x0 - halo + lx, nx), y = wrap_index(y0 - halo + ly, ny);
+            const int xm = x == 0 ? nx - 1 : x - 1, xp = x == nx - 1 ? 0 : x + 1;
+            const int ym = y == 0 ? ny - 1 : y - 1, yp = y == ny - 1 ? 0 : y + 1;
+            const size_t c0 = (size_t)x * a.cs, cm = (size_t)xm * a.cs, cp = (size_t)xp * a.cs;
+            const float is = a.inv_scale;
+            R f[9];
+            f[0] = load_pop<ST>(s + c0 + 0 * L + y, is);
+            f[1] = load_pop<ST>(s + cm + 1 * L + y, is);
+            f[2] = load_pop<ST>(s + c0 + 2 * L + ym, is);
+            f[3] = load_pop<ST>(s + cp + 3 * L + y, is);
+            f[4] = load_pop<ST>(s + c0 + 4 * L + yp, is);
+            f[5] = load_pop<ST>(s + cm + 5 * L + ym, is);
+            f[6] = load_pop<ST>(s + cp + 6 * L + ym, is);
+            f[7] = load_pop<ST>(s + cp + 7 * L + yp, is);
+            f[8] = load_pop<ST>(s + cm + 8 * L + yp, is);
+            collide_cell<MODEL, ST>(f, a);
+            settle(f);
+            R *m = mem + lx * 9 * H + ly;
+#pragma unroll
+            for (int q = 0; q < 9; ++q) m[q * H] = f[q];
+            if (halo == 1 && lag != nullptr) store(lag, lx, ly, f);
+        }
+    }
+    // levels 2 .. ns, each one cell smaller on every side: the even ones A, the odd ones B
+    auto level = [&](int k, auto odd, auto last) __attribute__((always_inline)) {
+        constexpr bool ODD = decltype(odd)::value, LAST = decltype(last)::value;
+        const int hk = h + 2 * (ns - k), n = (w + 2 * (ns - k)) * hk;
+        const float rh = 1.0f / float(hk);
+        for (int i = threadIdx.x; i < n; i += NT) {
+            const int ix = int((float(i) + 0.5f) * rh);
+            const int lx = ix + k - 1, ly = i - ix * hk + k - 1;
+            R *m = mem + lx * 9 * H + ly;
+            R f[9];
+#pragma unroll
+            for (int q = 0; q < 9; ++q)
+                f[q] = ODD ? m[opposite(q) * H] : m[(q - 9 * cx(q)) * H - cy(q)];
+            collide_cell<MODEL, ST>(f, a);
+            if constexpr (LAST) {
+                store(d, lx, ly, f);
+            } else {
+                settle(f);
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    if constexpr (ODD) m[q * H] = f[q];
+                    else m[(q - 9 * cx(q)) * H - cy(q)] = f[opposite(q)];
+                if (k == halo && lag != nullptr) store(lag, lx, ly, f);
+            }
+        }
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    for (int k = 2; k < ns; ++k) {
+        __syncthreads();
+        if (k & 1) level(k, yes, no);
+        else level(k, no, no);
+    }
+    __syncthreads();
+    if (ns & 1) level(ns, yes, yes);
+    else level(ns, no, yes);
+}
+
+}  // namespace plbm
