@@ -290,8 +290,9 @@ int plbm_pass(plbm_lattice *h, int model, int steps, int src, int dst);
 int plbm_get_steps_per_launch(const plbm_lattice *h, int model, int *steps);
 /* Work split of a pass (engine extension, no counterpart in the reference): each band of
  * 56 (F64 / F64S) or 48 (F32S / F16S) rows is cut into `segments` column ranges of nearly
- * equal length, one wavefront each; 0 = chosen from the grid (64 segments, each of at
- * least 8 columns).  Results do not depend on it.  The get variant reports the setting. */
+ * equal length, one wavefront each (a grid small enough for tiles then walks columns too);
+ * 0 = chosen from the grid (as many as fill the chip best, each of at least 8 columns).
+ * Results do not depend on it in F64 storage; the others agree to roundoff.  The get variant reports the setting. */
 int plbm_set_pass_segments(plbm_lattice *h, int segments);
 int plbm_get_pass_segments(const plbm_lattice *h, int *segments);
 /* Third population buffer of plbm_run / plbm_run_op in passes (engine extension, no

@@ -167,6 +167,7 @@ constexpr int kModels = 4;
 constexpr int kMaxStepsPerLaunch = 8;  // temporal-blocking depth of plbm_run
 int max_steps_per_pass(int storage);  // PLBM_BGK, PLBM_TRT, PLBM_RR, PLBM_BGK_SPLIT
 constexpr int kReduceBlocks = 1024;
+constexpr int kComputeUnits = 256;  // MI355X
 
 // Host plane of nx columns with pitch ld (ld >= ny, the host arrays of the upload /
 // download entry points) to / from a compact device plane (pitch ny), synchronous on

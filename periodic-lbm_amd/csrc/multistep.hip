@@ -5,7 +5,7 @@
 // lattice NS steps (NS = 2..8) and reads / writes every population once per pass:
 //
 //  * A wavefront owns 64 consecutive rows y and walks a segment of columns along x (by
-//    default 1/64 of the width, at least 8 columns).  Of its rows, VR produce output; NS
+//    default as many per band as fill the chip best, of at least 8 columns).  Of its rows, VR produce output; NS
 //    rows on each side are halo (VR + 2 NS <= 64).  VR is a multiple of 8 so that each
 //    wave's stores start and end on 64-byte boundaries.
 //  * Level k (k = 0 .. NS-1) keeps the pull-ready values of f^{n+k} for the last three
@@ -56,8 +56,19 @@ __device__ __forceinline__ int xcd_contiguous(int b, int nwg) {
     return x * base + min(x, rem) + b / 8;
 }
 
+// Wavefronts per SIMD asked of the compiler (1 = its own choice): the FP64 BGK passes of 8
+// steps need 4-6 registers beyond 256, and held to 256 (4-6 spilled) they run two wavefronts
+// per SIMD (4096^2, each at its best split: 939 -> 890 us; 2048^2 287 -> 275).  RR would
+// spill 42 (1487 -> 1573 us); held to three wavefronts the FP32 BGK and RR passes of 8 steps
+// spill 4-8 (2048^2 BGK 128 -> 151 us), those of 7 steps do not and are as fast.
 template <int MODEL, int ST, int NS>
-__global__ void __launch_bounds__(256) k_multi(StepArgs a, int waves_y, int m, int sync) {
+constexpr int pass_waves_per_eu() {
+    return ST == PLBM_F64 && NS == 8 && (MODEL == PLBM_BGK || MODEL == PLBM_BGK_SPLIT) ? 2 : 1;
+}
+
+template <int MODEL, int ST, int NS>
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(pass_waves_per_eu<MODEL, ST, NS>()))) k_multi(StepArgs a, int waves_y, int m, int sync) {
     // wave-uniform: the column walk's indices and addresses are then scalar
     const int wg = xcd_contiguous(blockIdx.x, gridDim.x);
     const int gw = __builtin_amdgcn_readfirstlane(wg * 4 + (threadIdx.x >> 6));
@@ -76,19 +87,52 @@ __global__ void __launch_bounds__(256) k_multi(StepArgs a, int waves_y, int m, i
 
 int max_steps_per_pass(int) { return kMaxPassSteps; }
 
-// Column segments per row band of a pass when the caller has not chosen: 64, each of at
-// least 8 columns.  Measured with 8 steps per pass (TRT, GLUPS for 48 / 64 / 96 segments
-// per band; FP64, FP32, FP16 storage): 8192^2 181 / 191 / 184, 351 / 366 / 358, 360 / 378
-// / 365; 4096^2 168 / 174 / 168, 305 / 326 / 316, 273 / 322 / 333; FP64 2048^2 (32 / 64
-// / 128) 145 / 154 / 136, 1024^2 84 / 102 / 94, 512^2 (16 / 32 / 64) 24 / 38 / 53.  With
-// fewer wavefronts than resident slots the short segments still pay: the pass is bound by
-// each wavefront's sequential walk.
-int default_pass_segments(int nx) { return std::max(1, std::min(64, nx / 8)); }
+// The split that decides whether single steps were the automatic choice (enough_walks).
+static int walk_segments(int nx) { return std::max(1, std::min(64, nx / 8)); }
+
+// Time of k layers of workgroups on a CU, each walking one column: k = 1 is one wavefront per
+// SIMD, `occ` layers run at once.  Fitted to walks of 1600^2 to 8192^2 (us per column at
+// 2048^2, 8 steps): FP64 TRT, two at once, 2.1 3.1 4.1 5.1 . 7.2 . 9.2 for k = 1..8, which
+// overlap from layer to layer; FP64 RR, one at once, proportional to k; FP32 / FP16 TRT,
+// three at once, 1.5 1.8 2.2 3.2 . 3.9, BGK, two at once, 1.9 2.2 3.6 3.8 . 5.3, in steps.
+static double walk_layers(int k, int occ, int bytes) {
+    if (bytes == 8) return occ >= 2 ? (1 + k) / 3.0 : 0.1 + k;
+    const int full = (k - 1) / occ, rest = (k - 1) % occ;
+    const double first = occ == 1 ? 1.0 : occ == 2 ? 0.87 : 0.7, turn = occ == 2 ? 0.78 : 0.9;
+    return turn * full + first + (occ > 1 ? (1 - first) * rest / (occ - 1) : 0.0);
+}
+
+// Column segments per row band of a pass when the caller has not chosen: of every count
+// that leaves at least 8 columns a segment, the one with the least layers x walk, the walk
+// being a segment's columns and its 2 NS start-up columns.  A fixed 64 leaves the last layer
+// nearly empty on many grids: us per pass, 64 / chosen: 1600^2 TRT FP64 8 steps 166 / 131;
+// 2048^2 BGK FP64 7 steps 220 / 205, FP32 8 steps 169 / 129; 4096^2 TRT FP64 711 / 663, FP32
+// 385 / 342; 8192^2 TRT FP64 2566 / 2539.  A TRT pass that also stores the lagged level gains
+// from the barrier per column that launch_multi gives it where all wavefronts walk alike
+// (8192^2, 8 steps, ms with 64 segments and the barrier / the best without: FP64 2.99 / 3.03,
+// FP32 1.59 / 1.66, FP16 1.51 / 1.97); BGK and RR, with more arithmetic per column, do not.
+static int pass_segments(int nx, int bands, int ns, int model, int bytes, int occ, bool lag) {
+    const double with_barrier =
+        model != PLBM_TRT ? 1.0 : bytes == 8 ? 0.975 : bytes == 4 ? 0.92 : 0.82;
+    int best = 1;
+    double cost = 1e300;
+    for (int m = 1; m <= std::max(1, std::min(256, nx / 8)); ++m) {
+        const long long wgs = ((long long)bands * m + 3) / 4;
+        const int k = (int)((wgs + kComputeUnits - 1) / kComputeUnits);
+        double c = walk_layers(k, occ, bytes) * ((nx + m - 1) / m + 2 * ns);
+        if (lag && nx % m == 0 && (long long)bands * m % 4 == 0) c *= with_barrier;
+        if (c < cost) {
+            cost = c;
+            best = m;
+        }
+    }
+    return best;
+}
 
 // Whether the default work split gives the column walk at least 512 wavefronts.
 static bool enough_walks(const plbm_lattice *h) {
     const int vr = multi_rows(storage_bytes(h->storage), kMaxPassSteps);
-    return (long)((h->ny + vr - 1) / vr) * default_pass_segments(h->nx) >= 512;
+    return (long)((h->ny + vr - 1) / vr) * walk_segments(h->nx) >= 512;
 }
 
 // Most steps of a launch of plbm_run when the caller has not chosen: 8 where it runs in
@@ -124,8 +168,20 @@ int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
                 if constexpr (NS <= max_steps_per_pass<SS>()) {
                     constexpr int vr = multi_vr<SS, NS>();
                     const int waves_y = (h->ny + vr - 1) / vr;
-                    const int m = h->pass_segs > 0 ? std::min(h->pass_segs, h->nx)
-                                                   : default_pass_segments(h->nx);
+                    // workgroups of this kernel that a CU holds at once (each one wavefront
+                    // per SIMD), asked of the runtime once
+                    static const int occ = [] {
+                        int n = 0;
+                        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                            &n, k_multi<MM, SS, NS>, 256, 0);
+                        if (e != hipSuccess) (void)hipGetLastError();
+                        return e == hipSuccess && n > 0 ? n : 2;
+                    }();
+                    const int m = h->pass_segs > 0
+                                      ? std::min(h->pass_segs, h->nx)
+                                      : pass_segments(h->nx, waves_y, NS, MM,
+                                                      (int)storage_bytes(h->storage), occ,
+                                                      lag != nullptr);
                     const long long nw = (long long)waves_y * m;
                     const dim3 grid((unsigned)((nw + 3) / 4));
                     // A barrier per column keeps a workgroup's four wavefronts (adjacent

@@ -54,22 +54,22 @@ double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
 }
 
 // Grids up to this many cells take tiles: about where the column walk catches up.  us per
-// step at both sides' automatic depths, column walk / tiles, FP64 | FP32 | FP16:
-//   BGK  1200^2 19.4/14.6 | 8.7/6.9 | 8.5/7.2;  1400^2 21.6/22.3 | 10.3/8.8 | 10.0/9.5;
-//        2048^2 41.7/44.1 | 22.0/21.9 | 21.8/18.6;  3000 x 1500 - | - | 17.2/19.6;
-//        3000^2 73.0/92.1 | 36.4/47.9 | 33.9/38.9
-//   TRT  1000^2 10.5/10.3 | 6.4/5.9 | 6.3/4.5;  1200^2 11.7/13.1 | 7.3/6.4 | 7.1/6.4;
-//        1600^2 21.2/32.6 | 11.1/12.6 | 11.1/10.0;  2048^2 26.1/40.8 | 14.9/20.9 | 13.8/15.7
-//   RR   1200^2 27.8/17.5 | 12.4/9.3 | 12.2/9.9;  2048^2 62.5/55.2 | 31.7/26.3 | 30.7/25.6;
-//        2600^2 98.0/84.8 | 43.4/43.0 | 42.4/39.8;  3000^2 110.9/114.2 | 50.8/57.7 | 48.5/53.0
+// step at both sides' automatic depths, column walk / tiles, FP64 | FP32 | FP16 (whose depth
+// stays 8, see run_steps):
+//   BGK   800^2 8.9/6.8 | 5.2/3.3 | 5.5/4.1;    1200^2 14.7/14.5 | 8.3/6.8 | 7.9/7.5;
+//        1400^2 18.0/21.2 | 10.0/8.7 | 10.1/9.9;  1600^2 22.1/33.5 | 11.7/14.0 | 12.2/12.1
+//   TRT   800^2 6.7/5.8 | 4.5/3.2 | 4.2/3.5;    1000^2 8.7/10.4 | 5.4/6.1 | 5.3/4.4;
+//        1200^2 11.2/13.3 | 7.0/6.5 | 6.7/6.2;  1400^2 13.0/19.9 | 8.3/8.2 | 7.9/8.0
+//   RR   1000^2 16.4/13.6 | 9.1/8.3 | 8.6/6.6;  1400^2 26.2/25.3 | 13.8/11.7 | 13.6/12.3;
+//        1600^2 32.2/36.4 | 16.8/18.8 | 16.3/15.7;  2048^2 50.8/54.5 | 25.1/25.3 | 23.1/24.6
 bool tile_cells(int storage, int model, long long cells) {
     const int bytes = (int)storage_bytes(storage);
     const auto pick = [&](long long f64, long long f32, long long f16) {
         return cells <= (bytes == 8 ? f64 : bytes == 4 ? f32 : f16);
     };
-    if (model == PLBM_TRT) return pick(1050000, 2000000, 2000000);
-    if (model == PLBM_RR) return pick(7000000, 7000000, 4200000);
-    return pick(1800000, 4000000, 4200000);
+    if (model == PLBM_TRT) return pick(850000, 1900000, 1700000);
+    if (model == PLBM_RR) return pick(2100000, 2200000, 2600000);
+    return pick(1400000, 2100000, 2400000);
 }
 
 // A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.

@@ -58,7 +58,6 @@ inline double tile_work(int shape, int ns, int w, int h) {
     return c;
 }
 constexpr double kTileLaunchWork = 2500;  // a launch and its ramp, in the same unit
-constexpr int kComputeUnits = 256;        // MI355X
 
 // The shape and depth (in [ns_min, ns_max]) that cost the least per step on an nx x ny
 // grid; returns the cost of a step.  The busiest CU sets the time: ceil(tiles / 256) tiles
