@@ -364,8 +364,10 @@ int plbm_batch_get_launch(const plbm_batch *b, int *ty, int *tx, int *resident_c
 int plbm_batch_set_steps_per_pass(plbm_batch *b, int steps);
 int plbm_batch_get_steps_per_pass(const plbm_batch *b, int *steps);
 /* Columns each wavefront of a pass walks (engine extension, no counterpart in the
- * reference): a case is cut into segments of this many columns.  Default 64; the
- * autotuner tries 16 to 256.  Results do not depend on it. */
+ * reference): a case is cut into segments of this many columns.  Until it is set (the
+ * getter then says 64) the engine chooses: LDS tiles for batches of few cells, else a length
+ * that fills the chip; the autotuner tries both and 16 to 256.  Results do not depend on it
+ * in F64 storage; the others agree to roundoff. */
 int plbm_batch_set_pass_columns(plbm_batch *b, int columns);
 int plbm_batch_get_pass_columns(const plbm_batch *b, int *columns);
 /* Autotuner: time `steps` (even) steps of every plan candidate (tile shapes, steps per

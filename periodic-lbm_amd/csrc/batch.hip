@@ -19,6 +19,9 @@
 //    wavefront per 56 x 64 (FP64, up to 4 steps) or 48 x 64 block of a case, listed in a
 //    wave table in place of the tile table.
 //
+//  * k_batch_tile (ns > 1, batches of few cells): the same passes in LDS tiles (tile.hpp),
+//    which fill the chip with fewer cells than the column walks do.
+//
 // Tile shape (ty, tx), steps per pass, columns per pass segment and the resident threshold
 // are picked by the project's autotuner (plbm_batch_autotune), which times candidates on a scratch copy of
 // the arena.
@@ -34,6 +37,7 @@
 #include "multistep.hpp"
 #include "reduce.hpp"
 #include "stepper.hpp"
+#include "tile.hpp"
 
 namespace plbm {
 
@@ -46,7 +50,9 @@ struct BatchCase {
 };
 
 struct BatchTile {
-    int c, x0, y0, n;  // case, first column, first row (row band with passes), columns
+    // case, first column, first row (row band with walks), columns (LDS tiles: columns +
+    // rows * 65536)
+    int c, x0, y0, n;
 };
 
 struct BatchCfg {
@@ -54,7 +60,9 @@ struct BatchCfg {
     int resident_cells = 0;    // cases with nx*ny <= this run in k_batch_resident
     int resident_block = 256;
     int ns = 1;                // steps per pass of the tiled cases (> 1: k_batch_multi)
-    int xs = kMultiXS;         // columns per wavefront segment of a pass
+    int xs = kMultiXS;         // columns per wavefront segment of a pass, as set
+    bool walk = false;         // xs was set: passes walk segments of xs columns
+    int shape = -1;            // LDS tile shape of the passes, -1: they walk (build_plan)
 };
 
 template <int ST>
@@ -138,6 +146,21 @@ __global__ void __launch_bounds__(256)
     a.src = parity ? base + c.elems : base;
     a.dst = parity ? base : base + c.elems;
     multi_wave<MODEL, ST, NS>(a, w.y0, w.x0, w.n);
+}
+
+// One pass of ns steps of every tiled case in LDS tiles.  parity 0: A -> B, 1: B -> A.
+template <int MODEL, int ST, class SHAPE>
+__global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4)))
+    k_batch_tile(const BatchCase *__restrict__ cases, const BatchTile *__restrict__ tiles,
+                 void *arena, int parity, int ns, float scale, float inv_scale) {
+    using T = typename Traits<ST>::T;
+    const BatchTile t = tiles[xcd_remap(blockIdx.x, gridDim.x)];
+    const BatchCase c = cases[t.c];
+    T *base = static_cast<T *>(arena) + c.off;
+    StepArgs a = case_args<ST>(c, scale, inv_scale);
+    a.src = parity ? base + c.elems : base;
+    a.dst = parity ? base : base + c.elems;
+    tile_steps<MODEL, ST, SHAPE>(a, ns, t.x0, t.n & 0xffff, t.y0, t.n >> 16);
 }
 
 // nsteps steps of one small case per workgroup; only workgroup barriers between steps.
@@ -302,9 +325,81 @@ static void drop_graphs(plbm_batch *b) {
     b->graphs.clear();
 }
 
-// Tile table and resident list for the current configuration.
-static int build_plan(plbm_batch *b, const BatchCfg &cfg, BatchTile **d_tiles, int *ntiles,
+// Batches of up to this many cells in passes take LDS tiles.  us per step in passes of 6,
+// sweeps of 32^2 to 512^2, walk / tiles at 0.7, 1.5, 2.7 and 4.8 M cells: FP64 TRT 8.0/6.9,
+// 15.5/12.8, 23.7/24.0, 35.5/43.9, BGK 9.0/8.0, 18.0/15.5, 27.2/26.9, 42.7/47.5, RR 13.7/11.7,
+// 26.8/22.4, 38.4/38.5, 65/63; FP32 TRT 4.7/4.1, 7.4/6.9, 10.8/11.1, 21.0/21.5 (FP16 alike),
+// RR 7.6/5.9, 13.7/10.9, 21.1/19.1, 33.3/30.3 and 59.6/57.3 at 10 M.  FP32 BGK walks: in
+// tiles it would take FP64 arithmetic (collide_tile) to keep its error.
+static bool batch_tile_cells(int storage, int model, long long cells) {
+    if (storage_bytes(storage) == 8)
+        return cells <= (model == PLBM_TRT ? 1600000 : model == PLBM_RR ? 2600000 : 2000000);
+    return cells <= (model == PLBM_TRT ? 2200000 : model == PLBM_RR ? 8000000 : 3000000);
+}
+
+// LDS tile shape of the passes of a plan, or -1 for column walks (larger batches, or the
+// caller set the walk's columns): the shape whose tiles cost the busiest CU the least.
+static int pass_shape(const plbm_batch *b, const BatchCfg &cfg) {
+    if (cfg.ns < 2 || cfg.walk || tile_wide(b->storage, b->model)) return -1;
+    long long cells = 0;
+    for (const BatchCase &k : b->cases)
+        if ((long long)k.nx * k.ny > cfg.resident_cells) cells += (long long)k.nx * k.ny;
+    if (!batch_tile_cells(b->storage, b->model, cells)) return -1;
+    int best = -1;
+    double cost = 1e300;
+    for (int s = 0; s < kTileShapes; ++s) {
+        int wx, wy;
+        tile_limits(s, cfg.ns, &wx, &wy);
+        double work = 0, n = 0;
+        for (const BatchCase &k : b->cases) {
+            if ((long long)k.nx * k.ny <= cfg.resident_cells) continue;
+            const int nbx = (k.nx + wx - 1) / wx, nby = (k.ny + wy - 1) / wy;
+            const double m = double(nbx) * nby;
+            n += m;
+            work += m * tile_work(s, cfg.ns, (k.nx + nbx - 1) / nbx, (k.ny + nby - 1) / nby);
+        }
+        const double c = n > 0 ? std::ceil(n / kComputeUnits) * work / n : 0;
+        if (c < cost) {
+            cost = c;
+            best = s;
+        }
+    }
+    return best;
+}
+
+// Columns of the walks' segments when the caller has not set them: the length with the least
+// layers of workgroups x walk (walk_layers), of 8 to 256.  us per step in passes of 6, 64
+// columns / chosen: FP32 BGK 18.3 / 9.2 at 1.5 M cells, 25.3 / 24.9 at 4.8 M, 67.8 / 66.0 at
+// 17.5 M; FP64 TRT 20.5 / 15.5, 35.4 / 35.5, 104 / 104.
+static int walk_columns(const plbm_batch *b, const BatchCfg &cfg) {
+    const int bytes = (int)storage_bytes(b->storage), vr = multi_rows(bytes, cfg.ns);
+    const int occ = bytes == 8 || (b->model != PLBM_TRT && cfg.ns > 6) ? 2 : 3;
+    int best = kMultiXS;
+    double cost = 1e300;
+    for (int xs = 8; xs <= 256; xs += xs < 64 ? 4 : 16) {
+        long long waves = 0;
+        int longest = 0;
+        for (const BatchCase &k : b->cases) {
+            if ((long long)k.nx * k.ny <= cfg.resident_cells) continue;
+            waves += (long long)((k.nx + xs - 1) / xs) * ((k.ny + vr - 1) / vr);
+            longest = std::max(longest, std::min(xs, k.nx));
+        }
+        if (waves == 0) break;
+        const int layers = (int)(((waves + 3) / 4 + kComputeUnits - 1) / kComputeUnits);
+        const double c = walk_layers(layers, occ, bytes) * (longest + 2 * cfg.ns);
+        if (c < cost) {
+            cost = c;
+            best = xs;
+        }
+    }
+    return best;
+}
+
+// Tile table and resident list for the current configuration; sets cfg.shape.
+static int build_plan(plbm_batch *b, BatchCfg &cfg, BatchTile **d_tiles, int *ntiles,
                       int **d_res, int *nres) {
+    cfg.shape = pass_shape(b, cfg);
+    const int xs = cfg.walk || cfg.ns < 2 ? cfg.xs : walk_columns(b, cfg);
     std::vector<int> order(b->ncases);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int i, int j) {
@@ -318,11 +413,22 @@ static int build_plan(plbm_batch *b, const BatchCfg &cfg, BatchTile **d_tiles, i
             res.push_back(c);
             continue;
         }
-        if (cfg.ns > 1) {  // wave table: {case, first column, row band, columns}
+        if (cfg.shape >= 0) {
+            int wx, wy;
+            tile_limits(cfg.shape, cfg.ns, &wx, &wy);
+            const int nbx = (k.nx + wx - 1) / wx, nby = (k.ny + wy - 1) / wy;
+            for (int i = 0; i < nbx; ++i)
+                for (int j = 0; j < nby; ++j) {
+                    const int x0 = part_start(k.nx, nbx, i), y0 = part_start(k.ny, nby, j);
+                    tiles.push_back({c, x0, y0,
+                                     (part_start(k.nx, nbx, i + 1) - x0) +
+                                         65536 * (part_start(k.ny, nby, j + 1) - y0)});
+                }
+        } else if (cfg.ns > 1) {  // wave table: {case, first column, row band, columns}
             const int vr = multi_rows(storage_bytes(b->storage), cfg.ns);
-            for (int x0 = 0; x0 < k.nx; x0 += cfg.xs)
+            for (int x0 = 0; x0 < k.nx; x0 += xs)
                 for (int wy = 0; wy * vr < k.ny; ++wy)
-                    tiles.push_back({c, x0, wy, std::min(cfg.xs, k.nx - x0)});
+                    tiles.push_back({c, x0, wy, std::min(xs, k.nx - x0)});
         } else {
             for (int x0 = 0; x0 < k.nx; x0 += cfg.tx)
                 for (int y0 = 0; y0 < k.ny; y0 += cfg.ty) tiles.push_back({c, x0, y0, 0});
@@ -356,7 +462,7 @@ static int build_plan(plbm_batch *b, const BatchCfg &cfg, BatchTile **d_tiles, i
     return PLBM_OK;
 }
 
-static int set_cfg(plbm_batch *b, const BatchCfg &cfg) {
+static int set_cfg(plbm_batch *b, BatchCfg cfg) {
     BatchTile *t = nullptr;
     int *r = nullptr;
     int nt = 0, nr = 0;
@@ -413,6 +519,18 @@ static int enqueue_steps(plbm_batch *b, void *arena, const BatchTile *tiles, int
                 // so the number of passes must have the parity of nsteps (as the resident
                 // cases, which flip once per step): split a pass in two when it has not
                 for (int d : pass_depths(cfg.ns, nsteps)) {
+                    if (cfg.shape >= 0) {
+                        PLBM_TRY(dispatch_tile_shape(cfg.shape, [&](auto sh) {
+                            using SH = decltype(sh);
+                            hipLaunchKernelGGL((k_batch_tile<MM, SS, SH>), dim3((unsigned)ntiles),
+                                               dim3(SH::T), 0, b->stream, b->d_cases, tiles, arena,
+                                               parity, d, sc, isc);
+                            PLBM_HIP(hipGetLastError());
+                            return PLBM_OK;
+                        }));
+                        parity ^= 1;
+                        continue;
+                    }
                     const dim3 grid((unsigned)((ntiles + 3) / 4));
                     auto go = [&](auto K) {
                         constexpr int NS = decltype(K)::value;
@@ -773,6 +891,7 @@ int plbm_batch_set_pass_columns(plbm_batch *b, int columns) try {
     PLBM_HIP(hipStreamSynchronize(b->stream));
     BatchCfg c = b->cfg;
     c.xs = columns;
+    c.walk = true;
     return set_cfg(b, c);
 } catch (...) {
     return plbm::host_exception();
@@ -883,13 +1002,16 @@ int plbm_batch_autotune(plbm_batch *b, int steps, double *best_ms) try {
             }
     const int max_ns = max_steps_per_pass(b->storage);
     for (int ns = 2; ns <= max_ns; ns += (ns < 4 ? 1 : 2))
-        for (int xs : {16, 32, 64, 128, 256})
+        for (int xs : {0, 16, 32, 64, 128, 256})  // 0: LDS tiles, where the batch takes them
             for (int res : {0, 4096, 16384, 36864})
                 for (int rb : {256, 1024}) {
                     if (res == 0 && rb != 256) continue;
                     BatchCfg c;
                     c.ns = ns;
-                    c.xs = xs;
+                    if (xs > 0) {
+                        c.xs = xs;
+                        c.walk = true;
+                    }
                     c.resident_cells = res;
                     c.resident_block = rb;
                     cands.push_back(c);
@@ -897,7 +1019,7 @@ int plbm_batch_autotune(plbm_batch *b, int steps, double *best_ms) try {
     BatchCfg best = b->cfg;
     double tbest = 1e300;
     int status = PLBM_OK;
-    for (const BatchCfg &c : cands) {
+    for (BatchCfg &c : cands) {
         BatchTile *t = nullptr;
         int *r = nullptr;
         int nt = 0, nr = 0;

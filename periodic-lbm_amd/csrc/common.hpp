@@ -211,13 +211,14 @@ namespace plbm {
 // column walks (multistep.hip), whichever suits the grid; with lag non-null it also stores
 // the state one step before the pass's last there.
 int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
-                 void *lag = nullptr, bool round_levels = false);
+                 void *lag = nullptr, bool as_single = false);
 // Tile passes (tile.hip): whether the lattice's passes run in tiles, and one such pass
-// (round_levels: FP16 storage rounds every level, as single steps do).
+// (as_single: with the roundings of single steps, FP16 storage at every level and FP32 BGK in
+// FP32 arithmetic; other passes round FP16 once and compute FP32 BGK in FP64).
 bool tile_grid(const plbm_lattice *h, int model);
 bool tile_cells(int storage, int model, long long cells);
 int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
-                bool round_levels);
+                bool as_single);
 double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
 // Run bookkeeping shared by the pass runs (multistep.hip): pass depths of a run, the
 // lattice's third buffer (nullptr when it cannot be allocated), and the final assignment

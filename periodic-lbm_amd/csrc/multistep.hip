@@ -90,18 +90,6 @@ int max_steps_per_pass(int) { return kMaxPassSteps; }
 // The split that decides whether single steps were the automatic choice (enough_walks).
 static int walk_segments(int nx) { return std::max(1, std::min(64, nx / 8)); }
 
-// Time of k layers of workgroups on a CU, each walking one column: k = 1 is one wavefront per
-// SIMD, `occ` layers run at once.  Fitted to walks of 1600^2 to 8192^2 (us per column at
-// 2048^2, 8 steps): FP64 TRT, two at once, 2.1 3.1 4.1 5.1 . 7.2 . 9.2 for k = 1..8, which
-// overlap from layer to layer; FP64 RR, one at once, proportional to k; FP32 / FP16 TRT,
-// three at once, 1.5 1.8 2.2 3.2 . 3.9, BGK, two at once, 1.9 2.2 3.6 3.8 . 5.3, in steps.
-static double walk_layers(int k, int occ, int bytes) {
-    if (bytes == 8) return occ >= 2 ? (1 + k) / 3.0 : 0.1 + k;
-    const int full = (k - 1) / occ, rest = (k - 1) % occ;
-    const double first = occ == 1 ? 1.0 : occ == 2 ? 0.87 : 0.7, turn = occ == 2 ? 0.78 : 0.9;
-    return turn * full + first + (occ > 1 ? (1 - first) * rest / (occ - 1) : 0.0);
-}
-
 // Column segments per row band of a pass when the caller has not chosen: of every count
 // that leaves at least 8 columns a segment, the one with the least layers x walk, the walk
 // being a segment's columns and its 2 NS start-up columns.  A fixed 64 leaves the last layer
@@ -143,9 +131,9 @@ int default_steps_per_launch(const plbm_lattice *h, int model) {
 }
 
 int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
-                 void *lag, bool round_levels) {
+                 void *lag, bool as_single) {
     if (ns >= 2 && ns <= kMaxPassSteps && tile_grid(h, model))
-        return launch_tile(h, model, ns, src, dst, lag, round_levels);
+        return launch_tile(h, model, ns, src, dst, lag, as_single);
     StepArgs a{};
     a.src = src;
     a.dst = dst;
@@ -301,14 +289,14 @@ static int timing_mark(plbm_lattice *h, int depth) {
 //
 // A grid that takes tiles chooses the depth itself when the caller has not
 // (plbm_set_steps_per_launch): the cheapest of 2..8 (pick_tile), spread evenly over the
-// passes.  FP16 storage rounds a state whenever it is stored, so there the depth shows in
-// the results: where single steps were the automatic choice before (grids of fewer than 512
-// column walks) every level is rounded as they round it, elsewhere the depth stays 8.
+// passes.  On grids of fewer than 512 column walks the passes stand for single steps and
+// round as they do (as_single).  On larger ones FP16 storage, which rounds a state whenever it
+// is stored, keeps the depth of 8.
 // While the stream is being captured, such small grids keep single steps: their slots do not
 // move, so that a caller's graph can be replayed.
 int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
     int ns = h->cfg[model].ns, lag_ns = h->cfg[model].lag_ns;
-    bool even = false, round_levels = false;
+    bool even = false, as_single = false;
     if (ns == 0) {
         const bool walks = enough_walks(h);
         ns = walks ? kMaxPassSteps : 1;
@@ -319,7 +307,7 @@ int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
                 int shape;
                 pick_tile(h->nx, h->ny, 2, kMaxPassSteps, &shape, &ns);
                 even = true;
-                round_levels = h->storage == PLBM_F16S;
+                as_single = !walks;
             }
         }
     }
@@ -338,7 +326,7 @@ int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
     void *aux = pass_aux(h);
     auto launch = [&](int k, void *lag) {
         PLBM_TRY(k == 1 ? launch_step(h, model, latest, other)
-                        : launch_multi(h, model, k, latest, other, lag, round_levels));
+                        : launch_multi(h, model, k, latest, other, lag, as_single));
         return timing_mark(h, k);
     };
     if (aux == nullptr) {

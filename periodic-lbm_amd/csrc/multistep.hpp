@@ -27,6 +27,18 @@ constexpr int max_steps_per_pass() {
     return kMaxPassSteps;
 }
 
+// Time of k layers of workgroups on a CU, each walking one column: k = 1 is one wavefront per
+// SIMD, `occ` layers run at once.  Fitted to walks of 1600^2 to 8192^2 (us per column at
+// 2048^2, 8 steps): FP64 TRT, two at once, 2.1 3.1 4.1 5.1 . 7.2 . 9.2 for k = 1..8, which
+// overlap from layer to layer; FP64 RR, one at once, proportional to k; FP32 / FP16 TRT,
+// three at once, 1.5 1.8 2.2 3.2 . 3.9, BGK, two at once, 1.9 2.2 3.6 3.8 . 5.3, in steps.
+inline double walk_layers(int k, int occ, int bytes) {
+    if (bytes == 8) return occ >= 2 ? (1 + k) / 3.0 : 0.1 + k;
+    const int full = (k - 1) / occ, rest = (k - 1) % occ;
+    const double first = occ == 1 ? 1.0 : occ == 2 ? 0.87 : 0.7, turn = occ == 2 ? 0.78 : 0.9;
+    return turn * full + first + (occ > 1 ? (1 - first) * rest / (occ - 1) : 0.0);
+}
+
 // Row y+1 / y-1 of a value held by every lane of a wavefront whose lane i holds row
 // base + i: DPP wave_shl:1 gives lane i the value of lane i+1, wave_shr:1 that of lane
 // i-1 (the edge lanes keep their own value; they are halo lanes of a pass).

@@ -18,19 +18,20 @@
 // 4.2.
 //
 // Per-cell arithmetic is collide_cell, as everywhere: FP64 results equal single steps bit
-// for bit, and the shifted FP64 / FP32 storages did on every case compared.
+// for bit, and the shifted FP64 / FP32 storages did on every case compared (but see
+// collide_tile for FP32 BGK).
 #include "tile.hpp"
 
 namespace plbm {
 
-template <int MODEL, int ST, class SHAPE>
+template <int MODEL, int ST, class SHAPE, bool WIDE>
 __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4)))
     k_tile(StepArgs a, int ns, int nbx, int nby) {
     const int b = xcd_remap(blockIdx.x, gridDim.x);  // neighbouring tiles share an L2
     const int by = b % nby, bx = b / nby;
     const int x0 = part_start(a.nx, nbx, bx), x1 = part_start(a.nx, nbx, bx + 1);
     const int y0 = part_start(a.ny, nby, by), y1 = part_start(a.ny, nby, by + 1);
-    tile_steps<MODEL, ST, SHAPE>(a, ns, x0, x1 - x0, y0, y1 - y0);
+    tile_steps<MODEL, ST, SHAPE, WIDE>(a, ns, x0, x1 - x0, y0, y1 - y0);
 }
 
 double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
@@ -62,6 +63,8 @@ double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
 //        1200^2 11.2/13.3 | 7.0/6.5 | 6.7/6.2;  1400^2 13.0/19.9 | 8.3/8.2 | 7.9/8.0
 //   RR   1000^2 16.4/13.6 | 9.1/8.3 | 8.6/6.6;  1400^2 26.2/25.3 | 13.8/11.7 | 13.6/12.3;
 //        1600^2 32.2/36.4 | 16.8/18.8 | 16.3/15.7;  2048^2 50.8/54.5 | 25.1/25.3 | 23.1/24.6
+// FP32 BGK in FP64 arithmetic (collide_tile): 512^2 4.4/2.7, 640^2 4.9/4.6, 800^2 5.3/4.9,
+// 1001 x 777 5.8/6.2, 1000^2 5.9/8.6.
 bool tile_cells(int storage, int model, long long cells) {
     const int bytes = (int)storage_bytes(storage);
     const auto pick = [&](long long f64, long long f32, long long f16) {
@@ -69,7 +72,7 @@ bool tile_cells(int storage, int model, long long cells) {
     };
     if (model == PLBM_TRT) return pick(850000, 1900000, 1700000);
     if (model == PLBM_RR) return pick(2100000, 2200000, 2600000);
-    return pick(1400000, 2100000, 2400000);
+    return pick(1400000, 700000, 2400000);
 }
 
 // A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.
@@ -78,7 +81,7 @@ bool tile_grid(const plbm_lattice *h, int model) {
 }
 
 int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
-                bool round_levels) {
+                bool as_single) {
     StepArgs a{};
     a.src = src;
     a.dst = dst;
@@ -93,7 +96,7 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
     a.lambda_odd_f = float(h->lambda_odd);
     a.scale = float(h->scale);
     a.inv_scale = float(1.0 / h->scale);
-    a.round_levels = round_levels;
+    a.round_levels = as_single && h->storage == PLBM_F16S;
     int shape = 0, wx, wy;
     pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
     tile_limits(shape, ns, &wx, &wy);
@@ -101,10 +104,17 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
     return dispatch_model(model, [&](auto M) {
         return dispatch_storage(h->storage, [&](auto S) {
             return dispatch_tile_shape(shape, [&](auto sh) {
+                constexpr int MM = decltype(M)::value, SS = decltype(S)::value;
                 using SH = decltype(sh);
-                hipLaunchKernelGGL((k_tile<decltype(M)::value, decltype(S)::value, SH>),
-                                   dim3((unsigned)(nbx * nby)), dim3(SH::T), 0, h->stream, a, ns,
-                                   nbx, nby);
+                auto go = [&](auto wide) {
+                    hipLaunchKernelGGL((k_tile<MM, SS, SH, decltype(wide)::value>),
+                                       dim3((unsigned)(nbx * nby)), dim3(SH::T), 0, h->stream, a,
+                                       ns, nbx, nby);
+                };
+                if (tile_wide(SS, MM) && !as_single)
+                    go(std::integral_constant<bool, tile_wide(SS, MM)>{});
+                else
+                    go(std::false_type{});
                 PLBM_HIP(hipGetLastError());
                 return PLBM_OK;
             });

@@ -85,9 +85,33 @@ __device__ __forceinline__ int wrap_index(int v, int n) {
     return v;
 }
 
+// One cell's collision in a tile.  WIDE (FP32 storage, BGK): in FP64 on the FP32 populations,
+// rounded once.  Where a tile replaces the column walk, whose FMAs the compiler places
+// differently at every level, the FP32 BGK arithmetic of single steps was 5-12% further off
+// the FP64 run (velocity after 300-600 steps at nu = 0.03: 9.3e-7 to 1.7e-6 against 8.1e-7 to
+// 1.5e-6); in FP64 it is 4.2e-8 to 4.6e-8.  Of the other FP32 collisions RR has the walk's
+// bits and TRT its error.
+template <int MODEL, int ST, bool WIDE>
+__device__ __forceinline__ void collide_tile(typename Traits<ST>::R (&f)[9], const StepArgs &a) {
+    if constexpr (WIDE) {
+        double g[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) g[q] = double(f[q]);
+        collide_bgk_shifted<double>(g, a.omega);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) f[q] = float(g[q]);
+    } else {
+        collide_cell<MODEL, ST>(f, a);
+    }
+}
+// Whether passes of this storage and model are WIDE where they do not stand for single steps.
+constexpr bool tile_wide(int storage, int model) {
+    return storage == PLBM_F32S && (model == PLBM_BGK || model == PLBM_BGK_SPLIT);
+}
+
 // The calling workgroup (SHAPE::T threads) advances cells [x0, x0 + w) x [y0, y0 + h) of
-// the grid described by `a` ns >= 2 steps, a.src -> a.dst, and, when a.lag is set, stores
-// the state one step before there.  w + 2 (ns - 1) <= XW, h + 2 (ns - 1) <= H.
+// the grid described by `a` ns >= 1 steps, a.src -> a.dst, and, when a.lag is set (ns >= 2),
+// stores the state one step before there.  w + 2 (ns - 1) <= XW, h + 2 (ns - 1) <= H.
 //
 // LDS holds one copy of the region's populations, updated in place.  A step pulls f_q(x)
 // from cell x - c_q, so writing the result where it was read from (A: the value of the
@@ -96,7 +120,7 @@ __device__ __forceinline__ int wrap_index(int v, int n) {
 // written back to (x, p)).  Every LDS word is read and written by the same thread in a
 // step, so that one barrier per step suffices, any number of cells per thread works, and
 // half the LDS of a ping-pong pair holds the tile.
-template <int MODEL, int ST, class SHAPE>
+template <int MODEL, int ST, class SHAPE, bool WIDE = false>
 __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, int w, int y0,
                                            int h) {
     using T = typename Traits<ST>::T;
@@ -146,7 +170,11 @@ __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, in
             f[6] = load_pop<ST>(s + cp + 6 * L + ym, is);
             f[7] = load_pop<ST>(s + cp + 7 * L + yp, is);
             f[8] = load_pop<ST>(s + cm + 8 * L + yp, is);
-            collide_cell<MODEL, ST>(f, a);
+            collide_tile<MODEL, ST, WIDE>(f, a);
+            if (halo == 0) {  // one step: nothing to hand on
+                store(d, lx, ly, f);
+                continue;
+            }
             settle(f);
             R *m = mem + lx * 9 * H + ly;
 #pragma unroll
@@ -167,7 +195,7 @@ __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, in
 #pragma unroll
             for (int q = 0; q < 9; ++q)
                 f[q] = ODD ? m[opposite(q) * H] : m[(q - 9 * cx(q)) * H - cy(q)];
-            collide_cell<MODEL, ST>(f, a);
+            collide_tile<MODEL, ST, WIDE>(f, a);
             if constexpr (LAST) {
                 store(d, lx, ly, f);
             } else {
@@ -180,6 +208,7 @@ __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, in
             }
         }
     };
+    if (halo == 0) return;
     constexpr std::true_type yes{};
     constexpr std::false_type no{};
     for (int k = 2; k < ns; ++k) {
