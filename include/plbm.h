@@ -168,7 +168,9 @@ int plbm_step_op(plbm_lattice *h, int op, int model, int src, int dst, double dt
 int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *iold, int *inew,
                 double dt);
 /* Pass depth of plbm_run_op: 1 = single fused steps, 2..3 = passes (FP64 storage only),
- * 0 = chosen from the grid size, operator and model.  The get variant reports the
+ * 0 = chosen from the grid size (FP64: passes of up to 6 steps, in LDS tiles on small grids
+ * and by column walks on larger ones; single steps on grids of fewer than 2048 walks of 64
+ * columns while the lattice's stream is being captured).  The get variant reports the
  * effective value for (op, model). */
 int plbm_set_op_steps_per_pass(plbm_lattice *h, int steps);
 int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model, int *steps);

@@ -90,32 +90,11 @@ int max_steps_per_pass(int) { return kMaxPassSteps; }
 // The split that decides whether single steps were the automatic choice (enough_walks).
 static int walk_segments(int nx) { return std::max(1, std::min(64, nx / 8)); }
 
-// Column segments per row band of a pass when the caller has not chosen: of every count
-// that leaves at least 8 columns a segment, the one with the least layers x walk, the walk
-// being a segment's columns and its 2 NS start-up columns.  A fixed 64 leaves the last layer
-// nearly empty on many grids: us per pass, 64 / chosen: 1600^2 TRT FP64 8 steps 166 / 131;
-// 2048^2 BGK FP64 7 steps 220 / 205, FP32 8 steps 169 / 129; 4096^2 TRT FP64 711 / 663, FP32
-// 385 / 342; 8192^2 TRT FP64 2566 / 2539.  A TRT pass that also stores the lagged level gains
-// from the barrier per column that launch_multi gives it where all wavefronts walk alike
-// (8192^2, 8 steps, ms with 64 segments and the barrier / the best without: FP64 2.99 / 3.03,
-// FP32 1.59 / 1.66, FP16 1.51 / 1.97); BGK and RR, with more arithmetic per column, do not.
-static int pass_segments(int nx, int bands, int ns, int model, int bytes, int occ, bool lag) {
-    const double with_barrier =
-        model != PLBM_TRT ? 1.0 : bytes == 8 ? 0.975 : bytes == 4 ? 0.92 : 0.82;
-    int best = 1;
-    double cost = 1e300;
-    for (int m = 1; m <= std::max(1, std::min(256, nx / 8)); ++m) {
-        const long long wgs = ((long long)bands * m + 3) / 4;
-        const int k = (int)((wgs + kComputeUnits - 1) / kComputeUnits);
-        double c = walk_layers(k, occ, bytes) * ((nx + m - 1) / m + 2 * ns);
-        if (lag && nx % m == 0 && (long long)bands * m % 4 == 0) c *= with_barrier;
-        if (c < cost) {
-            cost = c;
-            best = m;
-        }
-    }
-    return best;
-}
+// A TRT pass that also stores the lagged level gains from the barrier per column that
+// launch_multi gives it where all wavefronts walk alike (8192^2, 8 steps, ms with 64 segments
+// and the barrier / the best without: FP64 2.99 / 3.03, FP32 1.59 / 1.66, FP16 1.51 / 1.97);
+// BGK and RR, with more arithmetic per column, do not.
+static double barrier_gain(int bytes) { return bytes == 8 ? 0.975 : bytes == 4 ? 0.92 : 0.82; }
 
 // Whether the default work split gives the column walk at least 512 wavefronts.
 static bool enough_walks(const plbm_lattice *h) {
@@ -154,6 +133,7 @@ int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
             auto go = [&](auto K) {
                 constexpr int NS = decltype(K)::value;
                 if constexpr (NS <= max_steps_per_pass<SS>()) {
+                    using T = typename Traits<SS>::T;
                     constexpr int vr = multi_vr<SS, NS>();
                     const int waves_y = (h->ny + vr - 1) / vr;
                     // workgroups of this kernel that a CU holds at once (each one wavefront
@@ -167,9 +147,11 @@ int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
                     }();
                     const int m = h->pass_segs > 0
                                       ? std::min(h->pass_segs, h->nx)
-                                      : pass_segments(h->nx, waves_y, NS, MM,
+                                      : pass_segments(h->nx, waves_y, NS,
                                                       (int)storage_bytes(h->storage), occ,
-                                                      lag != nullptr);
+                                                      lag != nullptr && MM == PLBM_TRT
+                                                          ? barrier_gain((int)sizeof(T))
+                                                          : 1.0);
                     const long long nw = (long long)waves_y * m;
                     const dim3 grid((unsigned)((nw + 3) / 4));
                     // A barrier per column keeps a workgroup's four wavefronts (adjacent

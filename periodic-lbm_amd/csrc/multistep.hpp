@@ -39,6 +39,29 @@ inline double walk_layers(int k, int occ, int bytes) {
     return turn * full + first + (occ > 1 ? (1 - first) * rest / (occ - 1) : 0.0);
 }
 
+// Column segments per row band of a pass when the caller has not chosen: of every count
+// that leaves at least 8 columns a segment, the one with the least layers x walk, the walk
+// being a segment's columns and its 2 NS start-up columns.  A fixed 64 leaves the last layer
+// nearly empty on many grids: us per pass, 64 / chosen: 1600^2 TRT FP64 8 steps 166 / 131;
+// 2048^2 BGK FP64 7 steps 220 / 205, FP32 8 steps 169 / 129; 4096^2 TRT FP64 711 / 663, FP32
+// 385 / 342; 8192^2 TRT FP64 2566 / 2539.  `alike`: the factor on a pass's time where all
+// wavefronts walk the same number of columns.
+inline int pass_segments(int nx, int bands, int ns, int bytes, int occ, double alike) {
+    int best = 1;
+    double cost = 1e300;
+    for (int m = 1; m <= std::max(1, std::min(256, nx / 8)); ++m) {
+        const long long wgs = ((long long)bands * m + 3) / 4;
+        const int k = (int)((wgs + kComputeUnits - 1) / kComputeUnits);
+        double c = walk_layers(k, occ, bytes) * ((nx + m - 1) / m + 2 * ns);
+        if (nx % m == 0 && (long long)bands * m % 4 == 0) c *= alike;
+        if (c < cost) {
+            cost = c;
+            best = m;
+        }
+    }
+    return best;
+}
+
 // Row y+1 / y-1 of a value held by every lane of a wavefront whose lane i holds row
 // base + i: DPP wave_shl:1 gives lane i the value of lane i+1, wave_shr:1 that of lane
 // i-1 (the edge lanes keep their own value; they are halo lanes of a pass).

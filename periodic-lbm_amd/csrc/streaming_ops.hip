@@ -82,18 +82,24 @@ extern "C" int plbm_step_op(plbm_lattice *h, int op, int model, int src, int dst
     return plbm::host_exception();
 }
 
-// Steps per pass of plbm_run_op when the caller has not chosen, where the grid gives at
-// least 2048 wavefronts (FP64 storage; else single steps): 3, the most a pass holds
-// (8192^2, ms per step in passes of 2 / 3: FVM + BGK 1.68 / 1.66, FVM + TRT 1.35 / 1.35,
-// FDM + BGK 1.11 / 1.08, FDM + TRT 1.09 / 1.04, Sofonea + BGK 1.00 / 0.69; single steps
-// about 2.0).
-static int fd_steps_per_pass(const plbm_lattice *h, int op, int model) {
-    (void)op;
-    (void)model;
+// Whether single steps were the automatic choice before the passes could fill the chip on
+// grids of fewer than 2048 walks of 64 columns: while the stream is captured they still are,
+// as their slots do not move.
+static bool fd_few_walks(const plbm_lattice *h) {
+    return (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS) < 2048;
+}
+
+// Steps per pass of plbm_run_op when the caller has not chosen (FP64 storage; else single
+// steps): walks of 4, the most that fit (8192^2, ms per step with BGK in passes of 2 / 3 / 4:
+// FVM 1.22 / 1.20 / 1.16, FDM 1.04 / 0.96 / 0.89, Sofonea 0.95 / 0.74 / 0.67), or tiles of the
+// cheapest depth on small grids.
+static int fd_steps_per_pass(const plbm_lattice *h) {
     if (h->fd_ns > 0) return h->fd_ns;
     if (h->storage != PLBM_F64) return 1;
-    const long waves = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
-    return waves < 2048 ? 1 : 3;
+    if (!fd_tile_grid(h)) return kFdWalkSteps;
+    int shape, ns = 2;
+    pick_fd_tile(h->nx, h->ny, 2, kFdTileSteps, false, &shape, &ns);
+    return ns;
 }
 
 extern "C" int plbm_set_op_steps_per_pass(plbm_lattice *h, int steps) try {
@@ -110,7 +116,9 @@ extern "C" int plbm_set_op_steps_per_pass(plbm_lattice *h, int steps) try {
 extern "C" int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model,
                                           int *steps) try {
     PLBM_REQUIRE(h && steps, PLBM_ERR_ARG, "null argument");
-    *steps = fd_steps_per_pass(h, op, model);
+    (void)op;
+    (void)model;
+    *steps = fd_steps_per_pass(h);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();
@@ -125,7 +133,13 @@ extern "C" int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *
                  "unknown collision model " + std::to_string(model));
     PLBM_REQUIRE(h->params_set, PLBM_ERR_STATE, "plbm_set_params has not been called");
     if (op == PLBM_STREAM_EXACT) return plbm_run(h, model, nsteps, iold, inew);
-    const int ns = fd_steps_per_pass(h, op, model);
+    int ns = fd_steps_per_pass(h);
+    const bool even = h->fd_ns == 0 && fd_tile_grid(h);
+    if (h->fd_ns == 0 && ns > 1 && fd_few_walks(h)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
+        if (cap != hipStreamCaptureStatusNone) ns = 1;
+    }
     if (ns <= 1 || nsteps < 2) {
         for (int s = 0; s < nsteps; ++s) {
             PLBM_TRY(launch_fd(h, op, model, h->f[*iold], h->f[*inew], dt));
@@ -140,7 +154,9 @@ extern "C" int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *
     const int a0 = *iold, b0 = *inew;
     void *latest = h->f[a0], *other = h->f[b0];
     void *aux = pass_aux(h);
-    const std::vector<int> plan = aux ? lag_pass_plan(nsteps, ns) : pass_plan(nsteps - 1, ns);
+    const std::vector<int> plan = !aux   ? pass_plan(nsteps - 1, ns)
+                                  : even ? pass_plan(nsteps, ns)
+                                         : lag_pass_plan(nsteps, ns);
     for (size_t p = 0; p + 1 < plan.size(); ++p) {
         if (plan[p] == 1) PLBM_TRY(launch_fd(h, op, model, latest, other, dt));
         else PLBM_TRY(launch_fd_multi(h, op, model, plan[p], latest, other, dt));
