@@ -187,18 +187,21 @@ int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model, int *st
  *                       are on entry.  On return every slot holds what the reference's
  *                       buffer of the same index holds after the same steps (the caller
  *                       swaps its iold/inew ids once per step, as the reference does).
- *                       The last step moves 360 bytes per cell; the steps before it run in
- *                       temporally blocked passes (plbm_dugks_set_steps_per_pass).  The
- *                       two slots may exchange their device storage, so addresses from
+ *                       It runs in temporally blocked passes
+ *                       (plbm_dugks_set_steps_per_pass).  The two slots and the buffer of
+ *                       plbm_set_pass_lag_buffer may exchange their device storage (under
+ *                       stream capture the two slots only), so addresses from
  *                       plbm_buffer_ptr for them must be fetched again.  Asynchronous. */
 int plbm_dugks_collide(plbm_lattice *h, int src, int dst, double omega_full,
                        double omega_half);
 int plbm_dugks_stream(plbm_lattice *h, int src, int dst, double dt);
 int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, double dt,
                     double omega_full, double omega_half);
-/* Steps per pass of plbm_dugks_step: all steps but the last run in temporally blocked
- * passes of up to this many steps over device memory (1 = the collide + flux pair every
- * step; 2..3 = passes; 0 = chosen from the grid size).  Bit-identical for every value. */
+/* Steps per pass of plbm_dugks_step: 1 = the collide + flux pair every step; 2..3 = all
+ * steps but the last in temporally blocked passes of up to this many steps over device
+ * memory; 0 (default) = chosen from the grid size, the last pass also storing the
+ * half-collided state (plbm_set_pass_lag_buffer; without it, and under stream capture, as
+ * 2..3).  Bit-identical for every value.  The getter returns the depth for equal rates. */
 int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps);
 /* DUGKS as the reference builds it with -DDUGKS (src/periodic_dugks.F90:68,199,267,308):
  * the stream relaxes the interpolated face values of every face towards the face's own

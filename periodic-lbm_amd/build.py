@@ -46,10 +46,10 @@ CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fopenmp", "-Wa
 # with two wavefronts per SIMD; the ILP-maximising scheduler interleaves them better (the
 # arithmetic is unchanged; same-box A/B, TRT 8 steps per pass, GLUPS: 8192^2 FP64
 # 208.0 -> 212.4, FP16 storage 398.3 -> 403.6, FP32 386.0 -> 387.9; 4096^2 FP64 187.1 ->
-# 191.5; the DUGKS passes 32.3 -> 32.8).  For the batched and FV/FD kernels it measured
-# within -0.6 .. +0.3% and is not used.
+# 191.5).  For the batched kernels it measured within -0.6 .. +0.3%, and it slows DUGKS's
+# (2048^2 collide + flux 267 -> 306 us, passes of 3 81.3 -> 82.7 us per step): not used there.
 _MAX_ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
-HIP_EXTRA = {"multistep.hip": _MAX_ILP, "dugks.hip": _MAX_ILP}
+HIP_EXTRA = {"multistep.hip": _MAX_ILP}
 # Fortran shim modules in dependency order
 FORTRAN_SOURCES = [
     "plbm_capi.f90", "precision.F90", "fvm_bardow.F90", "periodic_lbm.f90",

@@ -17,11 +17,14 @@
 // The fused step (plbm_dugks_step) runs k_dugks_collide without the full collision
 // (\bar f^+ into the other slot) and k_dugks_flux with the collision recomputed from the
 // cell's own old populations, writing f^{n+1} over them in place: 360 bytes per cell per
-// step against 432 for the reference's copy + collide + stream sequence.  A run of several
-// steps does all but the last in temporally blocked passes (k_dugks_multi, up to three
-// steps per sweep, 144 bytes per cell per pass), and the two slots exchange their device
-// storage where needed, so that slot contents equal the reference's buffers after the
-// same number of perform_dugks_step calls.
+// step against 432 for the reference's copy + collide + stream sequence.
+//
+// plbm_dugks_step runs in passes of the FV/FD pass kernels (fd_ops.hpp, kOpDugks): 144 bytes
+// per cell and pass, 216 for the last, which also writes the half-collided state into the
+// lattice's third buffer; the three buffers' storage rotates so that slot contents equal the
+// reference's buffers after the same number of perform_dugks_step calls.  Without that buffer,
+// while the stream is captured, and when the caller set the pass depth, the last step is the
+// two-kernel form, the others passes, and the two slots exchange their storage at most.
 // The -DDUGKS build's form (half collision at 0.75 of its rate, which the caller passes,
 // and face collisions in the stream) is plbm_dugks_stream_faces / plbm_dugks_step_faces
 // (k_dugks_flux_faces), one collide + flux pair per step.
@@ -29,9 +32,11 @@
 #include <algorithm>
 #include <cmath>
 #include <utility>
+#include <vector>
 
 #include "common.hpp"
 #include "d2q9.hpp"
+#include "fd_ops.hpp"
 #include "multistep.hpp"
 #include "stepper.hpp"
 
@@ -229,98 +234,6 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// NS DUGKS steps per sweep over device memory (temporal blocking, as the pass kernel of
-// the lattice Boltzmann step): a wavefront owns 64 consecutive rows (56 with output, NS
-// halo rows on each side) and walks a strip of kMultiXS columns.  For every level k < NS
-// it keeps the half-collided state of the last three columns and the fully collided
-// state of the previous column in registers; when level k receives a column, level k+1
-// gets the column before it: the face values of that column (from the three-column
-// window, y-neighbours from the adjacent lanes) are subtracted from its full collision,
-// exactly as k_dugks_collide + k_dugks_flux do.  Only level NS is stored, so a pass
-// moves 144 bytes per cell for NS steps; the half-collided state is not materialised.
-template <int NS>
-__global__ void __launch_bounds__(256)
-    k_dugks_multi(const double *__restrict__ src, double *__restrict__ dst, int nx, int ny,
-                  int ldd, int waves_y, int nwaves, double dt, double om_full,
-                  double om_half) {
-    constexpr int VR = 56;
-    static_assert(VR + 2 * NS <= 64, "halo rows do not fit in a wavefront");
-    const int lane = threadIdx.x & 63;
-    const int gw = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (gw >= nwaves) return;  // the whole wavefront
-    const int wy = gw % waves_y, xsi = gw / waves_y;
-    const int r = VR * wy - NS + lane;  // unwrapped row of this lane
-    int y = r % ny;
-    if (y < 0) y += ny;
-    const bool out = lane >= NS && lane < VR + NS && r < ny;
-    const int x0 = xsi * kMultiXS;
-    const int ncols = min(kMultiXS, nx - x0);
-    const size_t L = (size_t)ldd, cs = 9 * L;
-    auto column = [&](int c) {
-        c %= nx;
-        if (c < 0) c += nx;
-        return (size_t)c * cs;
-    };
-    double H[NS][3][9];  // half-collided state, [level][newest column, -1, -2][q]
-    double F[NS][9];     // fully collided state of the newest column of each level
-#pragma unroll
-    for (int k = 0; k < NS; ++k)
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            F[k][q] = 0.0;
-#pragma unroll
-            for (int j = 0; j < 3; ++j) H[k][j][q] = 0.0;
-        }
-    double nxt[9];
-    {
-        const size_t cc = column(x0 - NS);
-#pragma unroll
-        for (int q = 0; q < 9; ++q) nxt[q] = src[cc + q * L + y];
-    }
-    const int iters = ncols + 2 * NS;
-    for (int i = 0; i < iters; ++i) {
-        double f[9];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) f[q] = nxt[q];
-        if (i + 1 < iters) {
-            const size_t cn = column(x0 - NS + i + 1);
-#pragma unroll
-            for (int q = 0; q < 9; ++q) nxt[q] = src[cn + q * L + y];
-        }
-#pragma unroll
-        for (int k = 0; k < NS; ++k) {
-            if (i < 2 * k) break;  // level k has no column yet
-            double h[9], b[9], bprev[9];
-#pragma unroll
-            for (int q = 0; q < 9; ++q) h[q] = b[q] = f[q];
-            dugks_bgk(h, om_half);
-            dugks_bgk(b, om_full);
-#pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                H[k][2][q] = H[k][1][q];
-                H[k][1][q] = H[k][0][q];
-                H[k][0][q] = h[q];
-                bprev[q] = F[k][q];
-                F[k][q] = b[q];
-            }
-            if (i < 2 * k + 2) break;  // level k+1 needs three columns of level k
-            f[0] = bprev[0];
-#pragma unroll
-            for (int q = 1; q < 9; ++q) {
-                const double fc = H[k][1][q], fe = H[k][0][q], fw = H[k][2][q];
-                f[q] = dugks_face_update(bprev[q], fc, fe, row_plus(fc), fw, row_minus(fc),
-                                         row_plus(fe), row_plus(fw), row_minus(fw),
-                                         row_minus(fe), dt * double(cx(q)), dt * double(cy(q)));
-            }
-            if (k + 1 == NS && out) {
-                const size_t co = (size_t)(x0 - 2 * NS + i) * cs;
-#pragma unroll
-                for (int q = 0; q < 9; ++q) __builtin_nontemporal_store(f[q], dst + co + q * L + y);
-            }
-        }
-    }
-}
-
 static int dugks_check(plbm_lattice *h, int a, int b) {
     PLBM_REQUIRE(h, PLBM_ERR_ARG, "null lattice handle");
     PLBM_REQUIRE(a >= 0 && a < h->nf && b >= 0 && b < h->nf && a != b, PLBM_ERR_ARG,
@@ -432,35 +345,48 @@ extern "C" int plbm_dugks_stream(plbm_lattice *h, int src, int dst, double dt) t
 
 namespace plbm {
 
-static int launch_dugks_multi(plbm_lattice *h, int ns, const double *src, double *dst,
-                              double dt, double om_full, double om_half) {
-    const int waves_y = (h->ny + 55) / 56;
-    const int nw = waves_y * ((h->nx + kMultiXS - 1) / kMultiXS);
-    const dim3 grid((unsigned)((nw + 3) / 4));
-    switch (ns) {
-    case 2:
-        hipLaunchKernelGGL(k_dugks_multi<2>, grid, dim3(256), 0, h->stream, src, dst, h->nx,
-                           h->ny, h->ldd, waves_y, nw, dt, om_full, om_half);
-        break;
-    case 3:
-        hipLaunchKernelGGL(k_dugks_multi<3>, grid, dim3(256), 0, h->stream, src, dst, h->nx,
-                           h->ny, h->ldd, waves_y, nw, dt, om_full, om_half);
-        break;
-    default:
-        set_error("DUGKS steps per pass must be 1..3");
-        return PLBM_ERR_ARG;
-    }
-    PLBM_HIP(hipGetLastError());
-    return PLBM_OK;
+// Equal rates (one formula, and equal for dt = 1; the same bits) need one collision and one
+// state per cell, others two of each, which fit less deep walks and small tiles only.  us per
+// step in the collide + flux pair / walks of 1, 2, 3 (without spills up to 3 and 1) / tiles:
+// equal rates 400^2 24 / 16.6, 13.3, 13.3 / 5.0, 1000^2 82 / 36, 23.4, 23.3 / 22.1, 1400^2
+// 138 / 62, 42.9, 40.4 / 37.4, 2048^2 267 / 116, 82, 81, 8192^2 4380 / 1860, 1203, 1127;
+// unequal 400^2 24 / 16.6, 17.1, 32 / 8.7, 1000^2 81 / 36, 30.6, 72 / 37.3, 2048^2 267 / 116,
+// 112, 347, 8192^2 4375 / 1856, 1560, 4608.
+constexpr int kDugksWalkOne = 3, kDugksWalkTwo = 2;
+constexpr long long kDugksTileCellsTwo = 500000;
+
+static bool dugks_tiles(const plbm_lattice *h, bool two) {
+    return two ? (long long)h->nx * h->ny <= kDugksTileCellsTwo : fd_tile_grid(h);
 }
 
-// Steps per pass of plbm_dugks_step when the caller has not chosen: 3 (measured best at
-// 8192^2: 2.06 ms per step against 2.18 for 2 and 4.37 for 1) where the grid gives at
-// least 2048 wavefronts, else 1.
-static int dugks_steps_per_pass(const plbm_lattice *h) {
+// Steps per pass: the caller's choice as far as the walks go, or the deepest walk, or tiles of
+// the cheapest depth.
+static int dugks_steps_per_pass(const plbm_lattice *h, bool two) {
+    const int walk = two ? kDugksWalkTwo : kDugksWalkOne;
+    if (!dugks_tiles(h, two)) return h->dugks_ns > 0 ? std::min(h->dugks_ns, walk) : walk;
     if (h->dugks_ns > 0) return h->dugks_ns;
-    const long waves = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
-    return waves >= 2048 ? 3 : 1;
+    int shape, ns = 2;
+    pick_fd_tile(h->nx, h->ny, 2, kFdTileSteps, two, &shape, &ns);
+    return ns;
+}
+
+// One pass of ns steps, src -> dst; with `half` set it also stores there the half-collided
+// state that the last step's fluxes came from.
+static int launch_dugks_pass(plbm_lattice *h, int ns, const double *src, double *dst,
+                             double *half, double dt, double om_full, double om_half) {
+    StepArgs a = fd_args(h, src, dst);
+    a.lag = half;
+    a.omega = om_full;
+    const FdScalars sc = fd_scalars(dt, om_half);
+    if (om_full == om_half) {
+        if (dugks_tiles(h, false)) return launch_fd_tile<kOpDugks, kDugksOne>(h, ns, a, sc);
+        if (ns == 1) return launch_fd_walk<kOpDugks, kDugksOne, 1>(h, a, sc);
+        if (ns == 2) return launch_fd_walk<kOpDugks, kDugksOne, 2>(h, a, sc);
+        return launch_fd_walk<kOpDugks, kDugksOne, kDugksWalkOne>(h, a, sc);
+    }
+    if (dugks_tiles(h, true)) return launch_fd_tile<kOpDugks, kDugksTwo>(h, ns, a, sc);
+    if (ns == 1) return launch_fd_walk<kOpDugks, kDugksTwo, 1>(h, a, sc);
+    return launch_fd_walk<kOpDugks, kDugksTwo, kDugksWalkTwo>(h, a, sc);
 }
 
 }  // namespace plbm
@@ -476,7 +402,7 @@ extern "C" int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps) try {
 
 extern "C" int plbm_dugks_get_steps_per_pass(const plbm_lattice *h, int *steps) try {
     PLBM_REQUIRE(h && steps, PLBM_ERR_ARG, "null argument");
-    *steps = dugks_steps_per_pass(h);
+    *steps = dugks_steps_per_pass(h, false);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();
@@ -489,19 +415,45 @@ extern "C" int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, 
     PLBM_REQUIRE(std::isfinite(dt) && std::isfinite(omega_full) && std::isfinite(omega_half),
                  PLBM_ERR_ARG, "non-finite dt or relaxation rate");
     if (nsteps == 0) return PLBM_OK;
-    // All steps but the last in passes of up to ns steps (f only); the last step with the
-    // collide + flux pair, which leaves the half-collided state in the other buffer.
-    const int ns = dugks_steps_per_pass(h);
+    const bool two = omega_full != omega_half;
+    const int ns = dugks_steps_per_pass(h, two);
     double *latest = static_cast<double *>(h->f[iold]);
     double *other = static_cast<double *>(h->f[inew]);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
+    const bool captured = cap != hipStreamCaptureStatusNone;
+    double *aux = h->dugks_ns == 0 && !captured ? static_cast<double *>(pass_aux(h)) : nullptr;
+    if (aux != nullptr) {
+        const std::vector<int> plan =
+            dugks_tiles(h, two) ? pass_plan(nsteps, ns) : lag_pass_plan(nsteps, ns);
+        for (size_t p = 0; p < plan.size(); ++p) {
+            const bool last = p + 1 == plan.size();
+            PLBM_TRY(launch_dugks_pass(h, plan[p], latest, other, last ? aux : nullptr, dt,
+                                       omega_full, omega_half));
+            std::swap(latest, other);
+        }
+        int a = iold, b = inew;
+        finish_run(h, iold, inew, nsteps, latest, aux, other, &a, &b);
+        return PLBM_OK;
+    }
+    // All steps but the last in groups, each of one pass, whose buffers change places, and
+    // for the steps that it does not reach the collide + flux pair, which stays in place; the
+    // last step is the pair, which leaves the half-collided state in the other buffer.  Where
+    // the slots' storage ends depends on the groups only, and a captured run's must not
+    // depend on more than the grid: single steps (in place) below 2048 walks of 64 columns.
+    const long walks = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
+    const int group = h->dugks_ns > 0 ? h->dugks_ns : !captured ? ns : walks < 2048 ? 1 : 3;
     for (int done = 0; done < nsteps - 1;) {
-        const int k = std::min(ns, nsteps - 1 - done);
-        if (k == 1) {
+        const int k = std::min(group, nsteps - 1 - done);
+        const int in_pass = k > 1 ? std::min(k, ns) : 0;
+        if (in_pass > 0) {
+            PLBM_TRY(launch_dugks_pass(h, in_pass, latest, other, nullptr, dt, omega_full,
+                                       omega_half));
+            std::swap(latest, other);
+        }
+        for (int j = in_pass; j < k; ++j) {
             launch_collide<false>(h, latest, other, nullptr, omega_full, omega_half);
             launch_flux<true>(h, other, latest, latest, dt, omega_full);
-        } else {
-            PLBM_TRY(launch_dugks_multi(h, k, latest, other, dt, omega_full, omega_half));
-            std::swap(latest, other);
         }
         done += k;
     }

@@ -98,3 +98,64 @@ def test_operator_runs_under_capture(P, gpu):
         torch.cuda.synchronize()
         ref.run_op("fvm_bardow", "trt", steps, 0, 1, 0.5)
         compare(lat, ref, (0, 1), (0, 1), ny, f"replay {replay}")
+
+
+RATES = {"equal": (0.4, 1.7, 1.7), "unequal": (0.7, 1.75, 1.6)}
+# 24 x 24 and 34 x 33 tiles; walks above 10^6 cells, or 5 10^5 at unequal rates
+DUGKS_GRIDS = EDGES + [(900, 613), LARGE]
+
+
+@pytest.mark.parametrize("rates", list(RATES))
+@pytest.mark.parametrize("nx,ny", DUGKS_GRIDS)
+def test_dugks_passes(P, gpu, nx, ny, rates):
+    """Automatic runs, whose last pass stores the half-collided state as well, and passes of a
+    chosen depth against the collide + flux pair."""
+    for depth, steps in ((0, 1), (0, 2), (0, 11), (2, 6), (3, 8)):
+        what = f"case dugks {rates} {nx}x{ny} passes of {depth}, {steps} steps"
+        print(what, flush=True)
+        lat, ref = lattice(P, nx, ny), lattice(P, nx, ny)
+        lat.dugks_set_steps_per_pass(depth)
+        ref.dugks_set_steps_per_pass(1)
+        lat.dugks_step(0, 1, steps, *RATES[rates])
+        ref.dugks_step(0, 1, steps, *RATES[rates])
+        compare(lat, ref, (0, 1), (0, 1), ny, what)
+
+
+@pytest.mark.parametrize("value", list(POISON))
+@pytest.mark.parametrize("rates", list(RATES))
+@pytest.mark.parametrize("nx,ny", [(70, 45), LARGE])
+def test_dugks_passes_of_values_out_of_range(P, gpu, nx, ny, rates, value):
+    poison = {(20, 30, 1): POISON[value], (0, 0, 2): POISON[value], (ny - 1, 33, 5): POISON[value]}
+    what = f"case dugks {rates} {value} {nx}x{ny}"
+    print(what, flush=True)
+    lat, ref = lattice(P, nx, ny, poison), lattice(P, nx, ny, poison)
+    ref.dugks_set_steps_per_pass(1)
+    lat.dugks_step(0, 1, 5, *RATES[rates])
+    ref.dugks_step(0, 1, 5, *RATES[rates])
+    compare(lat, ref, (0, 1), (0, 1), ny, what)
+
+
+@pytest.mark.parametrize("rates", list(RATES))
+def test_dugks_under_capture_and_without_third_buffer(P, gpu, rates):
+    import torch
+    nx, ny, steps = 96, 80, 6
+    lat, ref = lattice(P, nx, ny), lattice(P, nx, ny)
+    ref.dugks_set_steps_per_pass(1)
+    s = torch.cuda.Stream()
+    lat.set_stream(s.cuda_stream)
+    lat.dugks_step(0, 1, steps, *RATES[rates])
+    ref.dugks_step(0, 1, steps, *RATES[rates])
+    lat.sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        lat.dugks_step(0, 1, steps, *RATES[rates])
+    for replay in range(3):
+        with torch.cuda.stream(s):
+            g.replay()
+        torch.cuda.synchronize()
+        ref.dugks_step(0, 1, steps, *RATES[rates])
+        compare(lat, ref, (0, 1), (0, 1), ny, f"replay {replay}")
+    lat.set_pass_lag_buffer(False)
+    lat.dugks_step(0, 1, 7, *RATES[rates])
+    ref.dugks_step(0, 1, 7, *RATES[rates])
+    compare(lat, ref, (0, 1), (0, 1), ny, "two buffers")
