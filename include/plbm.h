@@ -384,10 +384,11 @@ int plbm_batch_autotune(plbm_batch *b, int steps, double *best_ms);
 /* ---------------------------------------------------------------- adjoint */
 
 /* Discrete adjoint of nsteps BGK steps (no counterpart in the reference).  Forward:
- * f^0 = feq(rho0, u0), f^{n+1} = collide_bgk(lbm_stream(f^n)) with the engine's fused
- * kernel; loss L = 1/2 sum_cells |u(f^N) - u*|^2, u = j/rho.  States are checkpointed
- * every checkpoint_every steps; the reverse sweep recomputes each segment and runs the
- * fused reverse kernel.  storage: PLBM_F64, PLBM_F64S or PLBM_F32S (FP32
+ * f^0 = feq(rho0, u0), f^{n+1} = collide_bgk(lbm_stream(f^n)) in passes of several steps
+ * with the roundings of single ones; loss L = 1/2 sum_cells |u(f^N) - u*|^2, u = j/rho.
+ * States are checkpointed every checkpoint_every steps; the reverse sweep recomputes each
+ * segment but the last, whose states the forward call keeps, and runs the reverse steps in
+ * passes of several as well.  storage: PLBM_F64, PLBM_F64S or PLBM_F32S (FP32
  * forward steps and checkpoints); the adjoint state is FP64 for every storage.  All field pointers are device pointers to (ny, nx) Fortran-order
  * FP64 arrays; the initial fields must stay valid until the backward call. */
 typedef struct plbm_adjoint plbm_adjoint;

@@ -1,6 +1,6 @@
 """Adjoint of the BGK stream-collide map, exposed to PyTorch.
 
-``Adjoint`` wraps plbm_adjoint_* (checkpointed forward, fused reverse kernel).
+``Adjoint`` wraps plbm_adjoint_* (checkpointed forward, reverse sweep in passes).
 ``VelocityMisfit`` is a torch.autograd.Function: loss = 1/2 sum |u(f^N) - u*|^2 after N
 BGK steps from f^0 = feq(1, u0), differentiable with respect to the initial velocity
 field (ux0, uy0) and the relaxation time tau (omega = 1/tau).

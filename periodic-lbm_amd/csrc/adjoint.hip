@@ -8,13 +8,17 @@
 //   mu      = J_C(g^n)^T lambda^{n+1}          (collision Jacobian at the pre-collision state)
 //   lambda^n_q(x - c_q) = mu_q(x)              (S^T: push streaming)
 //   dL/domega += sum_cells sum_q lambda^{n+1}_q (feq_q(g^n) - g^n_q)
-// and dL/du0, dL/drho0 = (d feq / d(rho, u))^T lambda^0.  One fused kernel does one reverse
-// step: it re-reads f^n with the forward's pull pattern, evaluates the Jacobian-transpose
-// product in registers and pushes mu to the neighbours.
+// and dL/du0, dL/drho0 = (d feq / d(rho, u))^T lambda^0.
 //
-// Memory: states are checkpointed every K steps during the forward sweep; the reverse
-// sweep recomputes each K-step segment from its checkpoint into a segment buffer, then
-// runs the K reverse steps.  Forward cost 2N - N/K steps, reverse N steps.
+// Memory: states are checkpointed every K steps during the forward sweep, which leaves the
+// last K-step segment's states in a segment buffer; the reverse sweep recomputes each earlier
+// segment into it from its checkpoint before it runs the K reverse steps.  Forward cost
+// about 2N - K steps, reverse N steps.
+//
+// All three run in LDS tiles of several steps: the forward from checkpoint to checkpoint
+// (tile.hip), the recomputation storing every level on its way, the reverse sweep in
+// k_adj_tile.  512^2 FP64, per step: forward 8.9 us in single steps -> 3.1, recomputation
+// 8.9 -> 4.0 (its writes at 4.7 TB/s), reverse 12.8 -> 7.0.
 //
 // For BGK with rho = sum g, u = sum c g / rho, feq_i = w_i rho (1 + P_i),
 // P_i = 3 c_i.u + 4.5 (c_i.u)^2 - 1.5 u.u:
@@ -30,36 +34,11 @@
 #include "common.hpp"
 #include "d2q9.hpp"
 #include "stepper.hpp"
+#include "tile.hpp"
 
 namespace plbm {
 
-int launch_step(plbm_lattice *h, int model, const void *src, void *dst);
 constexpr int kAdjBlocks = 2048;  // reduction partial slots (fixed => deterministic)
-
-template <class R>
-__device__ __forceinline__ void bgk_jacobian_t(const R g_unshifted_rho, const R ux, const R uy,
-                                               const R lam[9], R omega, R mu[9]) {
-    const R rho = g_unshifted_rho;
-    const R u2 = ux * ux + uy * uy;
-    R A = 0, Bx = 0, By = 0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        const R cu = R(cx(i)) * ux + R(cy(i)) * uy;
-        const R P = R(3) * cu + R(4.5) * cu * cu - R(1.5) * u2;
-        const R lw = lam[i] * R(wq(i));
-        A += lw * (R(1) + P);
-        const R t = R(3) + R(9) * cu;
-        Bx += lw * (t * R(cx(i)) - R(3) * ux);
-        By += lw * (t * R(cy(i)) - R(3) * uy);
-    }
-    Bx *= rho;
-    By *= rho;
-    const R inv = R(1) / rho;
-#pragma unroll
-    for (int j = 0; j < 9; ++j)
-        mu[j] = (R(1) - omega) * lam[j] +
-                omega * (A + (Bx * (R(cx(j)) - ux) + By * (R(cy(j)) - uy)) * inv);
-}
 
 // Macros of one stored cell (pulled or not) from its populations g (deviations
 // g_q = f_q - w_q for the shifted storages), in the adjoint's FP64 arithmetic.
@@ -85,11 +64,18 @@ __device__ __forceinline__ void cell_state(const double gs[9], double &rho, doub
 // rounding (500 reverse steps of FP32 would add about 1e-5 relative to the gradient)
 // drops out.
 
-// lambda^N and the loss of the final state.
+// Index of element q at x + c_q, periodic.
+__device__ __forceinline__ size_t neighbour(int x, int y, int q, int nx, int ny, int ldd) {
+    const int xq = x + cx(q), yq = y + cy(q);
+    return pop_index(q, xq < 0 ? nx - 1 : xq == nx ? 0 : xq, yq < 0 ? ny - 1 : yq == ny ? 0 : yq,
+                     ldd);
+}
+
+// lambda^N, stored as the mu that S^T would make it from, and the loss of the final state.
 template <int ST>
 __global__ void __launch_bounds__(256)
     k_adj_final(const void *fN, int nx, int ny, int ldd, float inv_scale, const double *uxt,
-                const double *uyt, double *lam, double *partials) {
+                const double *uyt, double *mu, double *partials) {
     using T = typename Traits<ST>::T;
     __shared__ double sh[256];
     double acc = 0.0;
@@ -110,7 +96,7 @@ __global__ void __launch_bounds__(256)
         const double inv = 1.0 / rho;
 #pragma unroll
         for (int q = 0; q < 9; ++q)
-            lam[c + (size_t)q * ldd] = (ex * (cx(q) - ux) + ey * (cy(q) - uy)) * inv;
+            mu[neighbour(x, y, q, nx, ny, ldd)] = (ex * (cx(q) - ux) + ey * (cy(q) - uy)) * inv;
     }
     sh[threadIdx.x] = acc;
     __syncthreads();
@@ -121,84 +107,232 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x == 0) partials[blockIdx.x] = sh[0];
 }
 
-// One reverse step: f^n (storage), lambda^{n+1} -> lambda^n, and the omega sensitivity
-// of this step accumulated into partials[blockIdx.x] (same slot every step: launches on
-// one stream are ordered, so the sum is race-free and deterministic).
-template <int ST>
-__global__ void __launch_bounds__(256)
-    k_adj_step(const void *fn, const double *__restrict__ lam_in, double *__restrict__ lam_out,
-               int nx, int ny, int ldd, double omega, float inv_scale, double *partials) {
-    using T = typename Traits<ST>::T;
-    __shared__ double sh[256];
-    double acc = 0.0;
-    const size_t n = (size_t)nx * ny;
-    const T *s = static_cast<const T *>(fn);
-    const size_t L = (size_t)ldd, cs = 9 * L;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int x = (int)(i / ny), y = (int)(i % ny);
-        const int xm = x == 0 ? nx - 1 : x - 1, xp = x == nx - 1 ? 0 : x + 1;
-        const int ym = y == 0 ? ny - 1 : y - 1, yp = y == ny - 1 ? 0 : y + 1;
-        const size_t c0 = (size_t)x * cs, cm = (size_t)xm * cs, cp = (size_t)xp * cs;
-        // g^n = S f^n at cell (x, y): the forward's pull pattern
-        double g[9];
-        g[0] = double(load_pop<ST>(s + c0 + 0 * L + y, inv_scale));
-        g[1] = double(load_pop<ST>(s + cm + 1 * L + y, inv_scale));
-        g[2] = double(load_pop<ST>(s + c0 + 2 * L + ym, inv_scale));
-        g[3] = double(load_pop<ST>(s + cp + 3 * L + y, inv_scale));
-        g[4] = double(load_pop<ST>(s + c0 + 4 * L + yp, inv_scale));
-        g[5] = double(load_pop<ST>(s + cm + 5 * L + ym, inv_scale));
-        g[6] = double(load_pop<ST>(s + cp + 6 * L + ym, inv_scale));
-        g[7] = double(load_pop<ST>(s + cp + 7 * L + yp, inv_scale));
-        g[8] = double(load_pop<ST>(s + cm + 8 * L + yp, inv_scale));
-        double rho, ux, uy, drho;
-        cell_state<Traits<ST>::shifted>(g, rho, ux, uy, drho);
-        double lam[9], mu[9];
+// One cell's reverse step: g = g^n, lam = lambda^{n+1} -> mu, and the cell's omega sensitivity
+// sum_q lambda_q (feq_q - g_q).  The sums over directions are those of six moments of
+// w_q lambda_q, and rho cancels from B_a / rho:
+//   A - m = 3 u.m1 + 4.5 u.m2.u - 1.5 u.u m,  B_a / rho = 3 m1_a + 9 (m2.u)_a - 3 u_a m,
+//   m = sum w_q lambda_q, m1_a = sum w_q lambda_q c_qa, m2_ab = sum w_q lambda_q c_qa c_qb,
+//   sum_q lambda_q feq_q = rho A  (in deviation form drho m + rho (A - m)),
+// a third of the operations of the sums written out.  FMAs are written where they are meant,
+// so that a cell's result does not depend on the kernel or level that computes it.
+template <bool SHIFTED>
+__device__ __forceinline__ double adj_cell(const double (&g)[9], const double (&lam)[9],
+                                           double omega, double (&mu)[9]) {
+#pragma clang fp contract(off)
+    const auto fma = [](double p, double q, double r) { return __builtin_fma(p, q, r); };
+    double d, jx, jy;
+    moments_shifted<double>(g, d, jx, jy);
+    const double rho = SHIFTED ? 1.0 + d : d, drho = SHIFTED ? d : d - 1.0;
+    const double inv = 1.0 / rho, ux = jx * inv, uy = jy * inv;
+    constexpr double w0 = wq(0), w1 = wq(1), w5 = wq(5);
+    const double s13 = lam[1] + lam[3], d13 = lam[1] - lam[3];
+    const double s24 = lam[2] + lam[4], d24 = lam[2] - lam[4];
+    const double s57 = lam[5] + lam[7], d57 = lam[5] - lam[7];
+    const double s68 = lam[6] + lam[8], d68 = lam[6] - lam[8];
+    const double wd = w5 * (s57 + s68);
+    const double m = fma(w0, lam[0], fma(w1, s13 + s24, wd));
+    const double mx = fma(w1, d13, w5 * (d57 - d68)), my = fma(w1, d24, w5 * (d57 + d68));
+    const double mxx = fma(w1, s13, wd), myy = fma(w1, s24, wd), mxy = w5 * (s57 - s68);
+    const double tx = fma(ux, mxx, uy * mxy), ty = fma(ux, mxy, uy * myy);
+    const double u2 = fma(ux, ux, uy * uy);
+    const double am = fma(3.0, fma(ux, mx, uy * my),
+                          fma(4.5, fma(ux, tx, uy * ty), -1.5 * u2 * m));  // A - m
+    const double m3 = -3.0 * m;
+    const double bx = fma(3.0, mx, fma(9.0, tx, ux * m3));  // B_a / rho
+    const double by = fma(3.0, my, fma(9.0, ty, uy * m3));
+    const double kx = omega * bx, ky = omega * by, rest = 1.0 - omega;
+    const double k0 = fma(omega, m + am, -fma(kx, ux, ky * uy));
+    const double kxp = k0 + kx, kxm = k0 - kx;
+    mu[0] = fma(rest, lam[0], k0);
+    mu[1] = fma(rest, lam[1], kxp);
+    mu[2] = fma(rest, lam[2], k0 + ky);
+    mu[3] = fma(rest, lam[3], kxm);
+    mu[4] = fma(rest, lam[4], k0 - ky);
+    mu[5] = fma(rest, lam[5], kxp + ky);
+    mu[6] = fma(rest, lam[6], kxm + ky);
+    mu[7] = fma(rest, lam[7], kxm - ky);
+    mu[8] = fma(rest, lam[8], kxp - ky);
+    double sg = 0.0;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) lam[q] = lam_in[c0 + (size_t)q * L + y];
-        // omega sensitivity: sum_q lambda_q (feq_q - g_q), in deviation form
-        double geq[9];
-        equilibrium_shifted<double>(drho, ux, uy, geq);
-        double d = 0;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const double gdev = Traits<ST>::shifted ? g[q] : g[q] - wq(q);
-            d += lam[q] * (geq[q] - gdev);
-        }
-        acc += d;
-        bgk_jacobian_t<double>(rho, ux, uy, lam, omega, mu);
-        // S^T: lambda^n_q(x - c_q, y - cy_q) = mu_q(x, y)
-        lam_out[c0 + 0 * L + y] = mu[0];
-        lam_out[cm + 1 * L + y] = mu[1];
-        lam_out[c0 + 2 * L + ym] = mu[2];
-        lam_out[cp + 3 * L + y] = mu[3];
-        lam_out[c0 + 4 * L + yp] = mu[4];
-        lam_out[cm + 5 * L + ym] = mu[5];
-        lam_out[cp + 6 * L + ym] = mu[6];
-        lam_out[cp + 7 * L + yp] = mu[7];
-        lam_out[cm + 8 * L + yp] = mu[8];
-    }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partials[blockIdx.x] += sh[0];
+    for (int q = 0; q < 9; ++q) sg = fma(lam[q], SHIFTED ? g[q] : g[q] - wq(q), sg);
+    return fma(drho, m, fma(rho, am, -sg));
 }
 
-// Gradient with respect to the initial macroscopic fields: f^0 = feq(rho0, u0).
+// Sum of many terms in two doubles (Knuth's two-sum): its error is of the order of the square
+// of a double's rounding, so that the total does not depend on how the steps are split into
+// passes and the grid into tiles.
+struct Sum2 {
+    double hi, lo;
+    __device__ __forceinline__ void add(double d) {
+#pragma clang fp contract(off)
+        const double s = hi + d, b = s - hi;
+        lo += (hi - (s - b)) + (d - b);
+        hi = s;
+    }
+    __device__ __forceinline__ void add(const Sum2 &o) {
+        add(o.hi);
+        lo += o.lo;
+    }
+    // an infinite sum's error term is NaN
+    __device__ __forceinline__ double value() const { return isfinite(hi) ? hi + lo : hi; }
+};
+// Sum over the calling workgroup of NT threads, valid in thread 0; sh holds NT / 64 values.
+template <int NT>
+__device__ __forceinline__ Sum2 block_sum(Sum2 v, Sum2 *sh) {
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) v.add({__shfl_xor(v.hi, st), __shfl_xor(v.lo, st)});
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int i = 1; i < NT / 64; ++i) v.add(sh[i]);
+    return v;
+}
+
+// ns reverse steps of one tile held in LDS, in place as tile_steps holds the forward ones
+// (tile.hpp), with every direction turned round: the adjoint state in memory is mu, before
+// S^T, so that level 1 pulls lambda_q(x) = mu_q(x + c_q) over the tile and its halo of ns - 1
+// cells; an even level gathers from (x + c_q, q) and leaves mu_p where the opposite direction
+// was read, an odd one reads (x, opposite(p)) and writes (x, p).  Level l takes g from state
+// top - (l - 1) stride, the last from `last`.  The omega sensitivity of the tile's own cells is
+// added to the thread's partial sum (a sum over the workgroup per pass took 3-4 us).
+//
+// Bound by its reads of the states, 1.5 times the tile's own with the halo: at 512^2 4.5 TB/s
+// from beyond the L2s, with 42% of the issue slots used.  The whole backward call, 500 steps at
+// 512^2, ms, in tiles S / M / L of 4 steps 6.7 / 6.5 / 6.7, of 8 steps 7.7 / 6.2 / 5.4 (L: one
+// tile per CU); 100 steps at 1024^2 5.8 - 6.2 from 4 steps on: the forward's choice of shape and
+// depth serves.  Loading a thread's next cell ahead, across the barriers, changed nothing (126
+// instead of 98 registers), nor did 32-bit offsets in FP64 (FP32 storage 4.4 -> 4.0 ms).
+template <int ST>
+struct AdjArgs {
+    using T = typename Traits<ST>::T;
+    const T *top, *last;
+    size_t stride, cs;
+    const double *mu_in;
+    double *mu_out;
+    Sum2 *partials;
+    int nx, ny, ldd;
+    double omega;
+    float inv_scale;
+};
+template <int ST, class SHAPE, bool FAR>
+__global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4)))
+    k_adj_tile(AdjArgs<ST> a, int ns, int nbx, int nby) {
+    using T = typename Traits<ST>::T;
+    using Offset = std::conditional_t<FAR, size_t, uint32_t>;  // bytes
+    constexpr int H = SHAPE::H, NT = SHAPE::T;
+    __shared__ double mem[SHAPE::XW * 9 * H];  // (lx, q, ly)
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int by = b % nby, bx = b / nby;
+    const int x0 = part_start(a.nx, nbx, bx), w = part_start(a.nx, nbx, bx + 1) - x0;
+    const int y0 = part_start(a.ny, nby, by), h = part_start(a.ny, nby, by + 1) - y0;
+    const int nx = a.nx, ny = a.ny, halo = ns - 1;
+    const size_t L = (size_t)a.ldd;
+    const uint32_t cs = (uint32_t)(a.cs * sizeof(T));  // bytes of a column
+    // Cell i of level k: in the tile's region, and its offsets and its neighbours' in a state.
+    struct Cell {
+        int lx, ly;
+        Offset c0, cm, cp, r0, rm, rp;
+    };
+    auto cell = [&](int k, int i, int hk, float rh) __attribute__((always_inline)) {
+        const int ix = int((float(i) + 0.5f) * rh);
+        Cell c;
+        c.lx = ix + k - 1;
+        c.ly = i - ix * hk + k - 1;
+        const int x = wrap_index(x0 + c.lx - halo, nx), y = wrap_index(y0 + c.ly - halo, ny);
+        c.c0 = FAR ? (Offset)x * cs : (Offset)__umul24(x, cs);
+        c.r0 = (Offset)y * sizeof(T);
+        const Offset xe = (Offset)(nx - 1) * cs, ye = (Offset)(ny - 1) * sizeof(T);
+        c.cm = x == 0 ? c.c0 + xe : c.c0 - cs;
+        c.cp = x == nx - 1 ? c.c0 - xe : c.c0 + cs;
+        c.rm = y == 0 ? c.r0 + ye : c.r0 - (Offset)sizeof(T);
+        c.rp = y == ny - 1 ? c.r0 - ye : c.r0 + (Offset)sizeof(T);
+        return c;
+    };
+    // q's population at x - c_q (S = 1) or x + c_q (-1)
+    auto from = [&](const Cell &c, int q, int S) __attribute__((always_inline)) {
+        const int dx = S * cx(q), dy = S * cy(q);
+        return (dx > 0 ? c.cm : dx < 0 ? c.cp : c.c0) + (dy > 0 ? c.rm : dy < 0 ? c.rp : c.r0);
+    };
+    auto mu_at = [&](auto *p, int q, Offset o) __attribute__((always_inline)) {
+        constexpr Offset wide = sizeof(double) / sizeof(T);
+        using C = std::conditional_t<std::is_const_v<std::remove_pointer_t<decltype(p)>>,
+                                     const char, char>;
+        return reinterpret_cast<decltype(p)>(reinterpret_cast<C *>(p + q * L) + wide * o);
+    };
+    Sum2 *mine = a.partials + (size_t)blockIdx.x * NT + threadIdx.x, sum = *mine;
+    auto level = [&](int k, auto first, auto odd) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first)::value, ODD = decltype(odd)::value;
+        const T *__restrict__ s = k == ns ? a.last : a.top - (size_t)(k - 1) * a.stride;
+        const int hk = h + 2 * (ns - k), n = (w + 2 * (ns - k)) * hk;
+        const float rh = 1.0f / float(hk);
+        for (int i = threadIdx.x; i < n; i += NT) {
+            double g[9], lam[9], mu[9];
+            const Cell c = cell(k, i, hk, rh);
+#pragma unroll
+            for (int q = 0; q < 9; ++q)
+                g[q] = double(load_pop<ST>(
+                    reinterpret_cast<const T *>(reinterpret_cast<const char *>(s + q * L) +
+                                                from(c, q, 1)),
+                    a.inv_scale));
+            double *m = mem + c.lx * 9 * H + c.ly;
+#pragma unroll
+            for (int q = 0; q < 9; ++q)
+                if constexpr (FIRST) lam[q] = *mu_at(a.mu_in, q, from(c, q, -1));
+                else lam[q] = ODD ? m[opposite(q) * H] : m[(q + 9 * cx(q)) * H + cy(q)];
+            const double d = adj_cell<Traits<ST>::shifted>(g, lam, a.omega, mu);
+            const int ox = c.lx - halo, oy = c.ly - halo;
+            const bool own = ox >= 0 && ox < w && oy >= 0 && oy < h;
+            if (own) sum.add(d);
+            if (k == ns) {
+                if (own)
+#pragma unroll
+                    for (int q = 0; q < 9; ++q) *mu_at(a.mu_out, q, c.c0 + c.r0) = mu[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 9; ++q)
+                    if constexpr (FIRST || ODD) m[q * H] = mu[q];
+                    else m[(q + 9 * cx(q)) * H + cy(q)] = mu[opposite(q)];
+            }
+        }
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    level(1, yes, no);
+    for (int k = 2; k <= ns; ++k) {
+        __syncthreads();
+        if (k & 1) level(k, no, yes);
+        else level(k, no, no);
+    }
+    *mine = sum;
+}
+
+// One partial sum per workgroup, or of one workgroup the total.
+__global__ void __launch_bounds__(256) k_adj_total(const Sum2 *in, size_t n, Sum2 *out,
+                                                   double *total) {
+    __shared__ Sum2 sh[4];
+    Sum2 v{0.0, 0.0};
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256)
+        v.add(in[i]);
+    v = block_sum<256>(v, sh);
+    if (threadIdx.x == 0) {
+        if (total) *total = v.value();
+        else out[blockIdx.x] = v;
+    }
+}
+
+// Gradient with respect to the initial macroscopic fields: f^0 = feq(rho0, u0),
+// lambda^0_q(x) = mu^0_q(x + c_q).
 __global__ void __launch_bounds__(256)
-    k_adj_initial(const double *lam0, int nx, int ny, int ldd, const double *rho0, const double *ux0,
+    k_adj_initial(const double *mu0, int nx, int ny, int ldd, const double *rho0, const double *ux0,
                   const double *uy0, double *grho, double *gux, double *guy) {
     const int y = blockIdx.x * blockDim.x + threadIdx.x, x = blockIdx.y;
     if (y >= ny) return;
-    const size_t i = (size_t)x * ny + y, c = pop_index(0, x, y, ldd);
+    const size_t i = (size_t)x * ny + y;
     const double rho = rho0[i], ux = ux0[i], uy = uy0[i], u2 = ux * ux + uy * uy;
     double gr = 0, gx = 0, gy = 0;
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
-        const double l = lam0[c + (size_t)q * ldd] * wq(q);
+        const double l = mu0[neighbour(x, y, q, nx, ny, ldd)] * wq(q);
         const double cu = cx(q) * ux + cy(q) * uy;
         gr += l * (1.0 + 3.0 * cu + 4.5 * cu * cu - 1.5 * u2);
         const double t = 3.0 + 9.0 * cu;
@@ -223,8 +357,8 @@ __global__ void __launch_bounds__(256) k_adj_sum(const double *partials, int n, 
     if (threadIdx.x == 0) *out = sh[0];
 }
 
-__global__ void __launch_bounds__(256) k_adj_zero(double *p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_adj_zero(double *p, size_t n) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0.0;
 }
 
@@ -236,12 +370,13 @@ struct plbm_adjoint {
     int nx = 0, ny = 0, storage = 0, nsteps = 0, every = 0, ncheck = 0;
     plbm_lattice *lat = nullptr;   // forward buffers (ping-pong) + launch plumbing
     void *checkpoints = nullptr;   // ncheck buffers: f^0, f^K, f^2K, ...
-    void *segment = nullptr;       // every buffers: states of one recomputed segment
-    void *lam[2] = {nullptr, nullptr};
-    size_t buf_bytes = 0, lam_bytes = 0;
+    void *segment = nullptr;       // every buffers: the states of one segment after its first
+    void *mu[2] = {nullptr, nullptr};
+    Sum2 *sums = nullptr;          // omega sensitivity, one per thread of a reverse pass
+    size_t nsums = 0;              // the most threads that one has
+    size_t buf_bytes = 0, mu_bytes = 0;
     double omega = 0;
     bool forward_done = false;
-    int final_buf = 0;             // lattice buffer holding f^N
     double *d_partials = nullptr;  // kAdjBlocks
     double *d_scalar = nullptr;    // 2
     const double *rho0 = nullptr, *ux0 = nullptr, *uy0 = nullptr;  // caller's device fields
@@ -258,8 +393,84 @@ static int adj_reduce_blocks(const plbm_adjoint *a) {
 static void *ckpt(plbm_adjoint *a, int k) {
     return static_cast<char *>(a->checkpoints) + (size_t)k * a->buf_bytes;
 }
-static void *seg(plbm_adjoint *a, int k) {
-    return static_cast<char *>(a->segment) + (size_t)k * a->buf_bytes;
+// f^{n0 + j} of segment k (n0 = k * every): its checkpoint or, once computed, from the buffer.
+static void *state(plbm_adjoint *a, int k, int j) {
+    return j == 0 ? ckpt(a, k) : static_cast<char *>(a->segment) + (size_t)(j - 1) * a->buf_bytes;
+}
+
+// Depth of the object's passes.
+static int adj_depth(const plbm_adjoint *a) {
+    int shape, ns = 1;
+    pick_tile(a->nx, a->ny, 1, kMaxStepsPerLaunch, &shape, &ns);
+    return ns;
+}
+// f^{n0+1} .. f^{n0+len} of segment k from its checkpoint.
+static int fill_segment(plbm_adjoint *a, int k, int len) {
+    if (len < 1) return PLBM_OK;
+    int j = 0;
+    for (int ns : pass_plan(len, adj_depth(a))) {
+        PLBM_TRY(launch_tile_levels(a->lat, ns, state(a, k, j), state(a, k, j + 1)));
+        j += ns;
+    }
+    return PLBM_OK;
+}
+// Tiles of a reverse pass of ns steps: shape, columns and rows of the grid of them.
+static void adj_tiles(const plbm_adjoint *a, int ns, int *shape, int *nbx, int *nby) {
+    int wx, wy;
+    pick_tile(a->nx, a->ny, ns, ns, shape, &ns);
+    tile_limits(*shape, ns, &wx, &wy);
+    *nbx = (a->nx + wx - 1) / wx;
+    *nby = (a->ny + wy - 1) / wy;
+}
+static size_t adj_threads(const plbm_adjoint *a, int ns) {
+    int shape = 0, nbx, nby;
+    adj_tiles(a, ns, &shape, &nbx, &nby);
+    const int t = dispatch_tile_shape(shape, [](auto s) { return decltype(s)::T; });
+    return (size_t)nbx * nby * t;
+}
+
+// One pass of ns reverse steps, states f^{top} (at `top`) down to the one at `last`.
+static int launch_adj(plbm_adjoint *a, int ns, const void *top, const void *last, const void *in,
+                      void *out) {
+    const plbm_lattice *h = a->lat;
+    int shape = 0, nbx, nby;
+    adj_tiles(a, ns, &shape, &nbx, &nby);
+    return dispatch_storage(a->storage, [&](auto S) {
+        constexpr int SS = decltype(S)::value;
+        if constexpr (SS == PLBM_F16S) {
+            return PLBM_ERR_ARG;  // refused by plbm_adjoint_create
+        } else {
+            using T = typename Traits<SS>::T;
+            AdjArgs<SS> g;
+            g.top = static_cast<const T *>(top);
+            g.last = static_cast<const T *>(last);
+            g.stride = h->elems;
+            g.cs = (size_t)9 * h->ldd;
+            g.mu_in = static_cast<const double *>(in);
+            g.mu_out = static_cast<double *>(out);
+            g.partials = a->sums;
+            g.nx = a->nx;
+            g.ny = a->ny;
+            g.ldd = h->ldd;
+            g.omega = a->omega;
+            g.inv_scale = float(1.0 / h->scale);
+            // byte offsets within a state in 32 bits, columns multiplied in 24
+            const bool near = h->elems * sizeof(double) < (1ull << 32) &&
+                              g.cs * sizeof(T) < (1u << 24) && a->nx < (1 << 24);
+            return dispatch_tile_shape(shape, [&](auto sh) {
+                using SH = decltype(sh);
+                auto go = [&](auto far_) {
+                    hipLaunchKernelGGL((k_adj_tile<SS, SH, decltype(far_)::value>),
+                                       dim3((unsigned)(nbx * nby)), dim3(SH::T), 0, a->stream, g,
+                                       ns, nbx, nby);
+                };
+                if (near) go(std::false_type{});
+                else go(std::true_type{});
+                PLBM_HIP(hipGetLastError());
+                return PLBM_OK;
+            });
+        }
+    });
 }
 
 }  // namespace plbm
@@ -288,7 +499,9 @@ int plbm_adjoint_create(int nx, int ny, int storage, int nsteps, int checkpoint_
     }
     a->stream = a->lat->stream;
     a->buf_bytes = a->lat->elems * storage_bytes(storage);
-    a->lam_bytes = a->lat->elems * sizeof(double);  // FP64 adjoint state for every storage
+    a->mu_bytes = a->lat->elems * sizeof(double);  // FP64 adjoint state for every storage
+    for (int ns = 1; ns <= adj_depth(a); ++ns)
+        a->nsums = std::max(a->nsums, adj_threads(a, ns));
     auto fail = [&](const char *m) {
         (void)hipGetLastError();
         set_error(m);
@@ -299,8 +512,9 @@ int plbm_adjoint_create(int nx, int ny, int storage, int nsteps, int checkpoint_
         return fail("hipMalloc of adjoint checkpoints failed");
     if (hipMalloc(&a->segment, a->every * a->buf_bytes) != hipSuccess)
         return fail("hipMalloc of the adjoint segment buffer failed");
-    if (hipMalloc(&a->lam[0], a->lam_bytes) != hipSuccess ||
-        hipMalloc(&a->lam[1], a->lam_bytes) != hipSuccess)
+    if (hipMalloc(&a->mu[0], a->mu_bytes) != hipSuccess ||
+        hipMalloc(&a->mu[1], a->mu_bytes) != hipSuccess ||
+        hipMalloc(&a->sums, a->nsums * sizeof(Sum2)) != hipSuccess)
         return fail("hipMalloc of adjoint buffers failed");
     if (hipMalloc(&a->d_partials, kAdjBlocks * sizeof(double)) != hipSuccess ||
         hipMalloc(&a->d_scalar, 2 * sizeof(double)) != hipSuccess)
@@ -316,8 +530,9 @@ int plbm_adjoint_destroy(plbm_adjoint *a) try {
     if (a->stream) (void)hipStreamSynchronize(a->stream);
     if (a->checkpoints) (void)hipFree(a->checkpoints);
     if (a->segment) (void)hipFree(a->segment);
-    for (void *p : a->lam)
+    for (void *p : a->mu)
         if (p) (void)hipFree(p);
+    if (a->sums) (void)hipFree(a->sums);
     if (a->d_partials) (void)hipFree(a->d_partials);
     if (a->d_scalar) (void)hipFree(a->d_scalar);
     if (a->lat) plbm_destroy(a->lat);
@@ -348,15 +563,22 @@ int plbm_adjoint_forward_dev(plbm_adjoint *a, const double *rho0, const double *
     a->ux0 = ux0;
     a->uy0 = uy0;
     PLBM_TRY(plbm_equilibrium_init_dev(h, 0, rho0, ux0, uy0));
-    int cur = 0;
-    for (int n = 0; n < a->nsteps; ++n) {
-        if (n % a->every == 0)
-            PLBM_HIP(hipMemcpyAsync(ckpt(a, n / a->every), h->f[cur], a->buf_bytes,
-                                    hipMemcpyDeviceToDevice, a->stream));
-        PLBM_TRY(launch_step(h, PLBM_BGK, h->f[cur], h->f[cur ^ 1]));
-        cur ^= 1;
+    // each segment in tile passes from its checkpoint to the next; the last one's states, f^N
+    // the last of them, stay in the segment buffer for the reverse sweep
+    const int depth = adj_depth(a);
+    const void *cur = h->f[0];
+    PLBM_HIP(hipMemcpyAsync(ckpt(a, 0), cur, a->buf_bytes, hipMemcpyDeviceToDevice, a->stream));
+    for (int k = 0; k + 1 < a->ncheck; ++k) {
+        const std::vector<int> plan = pass_plan(a->every, depth);
+        for (size_t p = 0; p < plan.size(); ++p) {
+            void *to = p + 1 == plan.size() ? ckpt(a, k + 1) : cur == h->f[0] ? h->f[1] : h->f[0];
+            PLBM_TRY(launch_tile(h, PLBM_BGK, plan[p], cur, to, nullptr, true));
+            cur = to;
+        }
     }
-    a->final_buf = cur;
+    const int len = a->nsteps - (a->ncheck - 1) * a->every;
+    PLBM_TRY(fill_segment(a, a->ncheck - 1, len));
+    cur = state(a, a->ncheck - 1, len);
     // loss and lambda^N
     const int nb = adj_reduce_blocks(a);
     PLBM_TRY(dispatch_storage(a->storage, [&](auto S) {
@@ -365,9 +587,9 @@ int plbm_adjoint_forward_dev(plbm_adjoint *a, const double *rho0, const double *
             set_error("adjoint: FP16 storage is not supported");
             return PLBM_ERR_ARG;
         } else {
-            hipLaunchKernelGGL(k_adj_final<SS>, dim3(nb), dim3(256), 0, a->stream, h->f[cur], a->nx,
+            hipLaunchKernelGGL(k_adj_final<SS>, dim3(nb), dim3(256), 0, a->stream, cur, a->nx,
                                a->ny, h->ldd, float(1.0 / h->scale), uxt, uyt,
-                               static_cast<double *>(a->lam[0]), a->d_partials);
+                               static_cast<double *>(a->mu[0]), a->d_partials);
             PLBM_HIP(hipGetLastError());
             return PLBM_OK;
         }
@@ -387,42 +609,34 @@ int plbm_adjoint_backward_dev(plbm_adjoint *a, double *grho0, double *gux0, doub
     PLBM_REQUIRE(a && gux0 && guy0 && gomega, PLBM_ERR_ARG, "null argument");
     PLBM_REQUIRE(a->forward_done, PLBM_ERR_STATE, "run plbm_adjoint_forward_dev first");
     plbm_lattice *h = a->lat;
-    const int nb = adj_reduce_blocks(a);
-    hipLaunchKernelGGL(k_adj_zero, dim3((nb + 255) / 256), dim3(256), 0, a->stream, a->d_partials,
-                       nb);
+    hipLaunchKernelGGL(k_adj_zero, dim3((unsigned)((2 * a->nsums + 255) / 256)), dim3(256), 0,
+                       a->stream, reinterpret_cast<double *>(a->sums), 2 * a->nsums);
     PLBM_HIP(hipGetLastError());
-    int cur = 0;  // lam[cur] holds lambda^{n+1}
+    const int depth = adj_depth(a);
+    int cur = 0;  // mu[cur] holds the adjoint state
     for (int k = a->ncheck - 1; k >= 0; --k) {
         const int n0 = k * a->every, n1 = std::min(a->nsteps, n0 + a->every);
-        // recompute f^{n0} .. f^{n1-1} into the segment buffer
-        PLBM_HIP(hipMemcpyAsync(seg(a, 0), ckpt(a, k), a->buf_bytes, hipMemcpyDeviceToDevice,
-                                a->stream));
-        for (int n = n0 + 1; n < n1; ++n)
-            PLBM_TRY(launch_step(h, PLBM_BGK, seg(a, n - 1 - n0), seg(a, n - n0)));
-        for (int n = n1 - 1; n >= n0; --n) {
-            PLBM_TRY(dispatch_storage(a->storage, [&](auto S) {
-                constexpr int SS = decltype(S)::value;
-                if constexpr (SS == PLBM_F16S) {
-                    return PLBM_ERR_ARG;
-                } else {
-                    hipLaunchKernelGGL(k_adj_step<SS>, dim3(nb), dim3(256), 0, a->stream,
-                                       seg(a, n - n0), static_cast<const double *>(a->lam[cur]),
-                                       static_cast<double *>(a->lam[cur ^ 1]), a->nx, a->ny,
-                                       h->ldd, a->omega, float(1.0 / h->scale), a->d_partials);
-                    PLBM_HIP(hipGetLastError());
-                    return PLBM_OK;
-                }
-            }));
+        if (k + 1 < a->ncheck) PLBM_TRY(fill_segment(a, k, n1 - n0 - 1));
+        int top = n1 - 1 - n0;
+        for (int ns : pass_plan(n1 - n0, depth)) {
+            PLBM_TRY(launch_adj(a, ns, state(a, k, top), state(a, k, top - ns + 1), a->mu[cur],
+                                a->mu[cur ^ 1]));
             cur ^= 1;
+            top -= ns;
         }
     }
-    // lam[cur] = lambda^0 -> gradients of the initial fields
+    // lambda^0 -> gradients of the initial fields
     hipLaunchKernelGGL(k_adj_initial, dim3((a->ny + 255) / 256, a->nx), dim3(256), 0, a->stream,
-                       static_cast<const double *>(a->lam[cur]), a->nx, a->ny, h->ldd, a->rho0,
+                       static_cast<const double *>(a->mu[cur]), a->nx, a->ny, h->ldd, a->rho0,
                        a->ux0, a->uy0, grho0, gux0, guy0);
     PLBM_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_adj_sum, dim3(1), dim3(256), 0, a->stream, a->d_partials, nb,
-                       a->d_scalar + 1);
+    Sum2 *part = reinterpret_cast<Sum2 *>(a->d_partials);
+    const int blocks = (int)std::min<size_t>(kAdjBlocks / 2, (a->nsums + 1023) / 1024);
+    hipLaunchKernelGGL(k_adj_total, dim3(blocks), dim3(256), 0, a->stream, a->sums, a->nsums, part,
+                       nullptr);
+    PLBM_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_adj_total, dim3(1), dim3(256), 0, a->stream, part, (size_t)blocks,
+                       nullptr, a->d_scalar + 1);
     PLBM_HIP(hipGetLastError());
     PLBM_HIP(hipMemcpyAsync(gomega, a->d_scalar + 1, sizeof(double), hipMemcpyDeviceToHost,
                             a->stream));

@@ -124,6 +124,8 @@ struct StepArgs {
     void *lag = nullptr;
     // Tile passes in FP16 storage: round every level to the storage, as single steps do.
     int round_levels = 0;
+    // Tile passes that keep every level: level k goes to dst + (k - 1) * level_stride elements.
+    size_t level_stride = 0;
 };
 
 // Strip length (columns per thread) of the stencil kernels that walk along x with a
@@ -219,6 +221,9 @@ bool tile_grid(const plbm_lattice *h, int model);
 bool tile_cells(int storage, int model, long long cells);
 int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
                 bool as_single);
+// One pass of ns >= 1 BGK steps that stores every level (F64, F64S, F32S storage), the roundings
+// of single steps: level k into the k-th of ns consecutive buffers at dst.
+int launch_tile_levels(plbm_lattice *h, int ns, const void *src, void *dst);
 double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
 // Run bookkeeping shared by the pass runs (multistep.hip): pass depths of a run, the
 // lattice's third buffer (nullptr when it cannot be allocated), and the final assignment

@@ -24,14 +24,14 @@
 
 namespace plbm {
 
-template <int MODEL, int ST, class SHAPE, bool WIDE>
+template <int MODEL, int ST, class SHAPE, bool WIDE, bool KEEP = false>
 __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4)))
     k_tile(StepArgs a, int ns, int nbx, int nby) {
     const int b = xcd_remap(blockIdx.x, gridDim.x);  // neighbouring tiles share an L2
     const int by = b % nby, bx = b / nby;
     const int x0 = part_start(a.nx, nbx, bx), x1 = part_start(a.nx, nbx, bx + 1);
     const int y0 = part_start(a.ny, nby, by), y1 = part_start(a.ny, nby, by + 1);
-    tile_steps<MODEL, ST, SHAPE, WIDE>(a, ns, x0, x1 - x0, y0, y1 - y0);
+    tile_steps<MODEL, ST, SHAPE, WIDE, KEEP>(a, ns, x0, x1 - x0, y0, y1 - y0);
 }
 
 double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
@@ -80,8 +80,7 @@ bool tile_grid(const plbm_lattice *h, int model) {
     return h->pass_segs == 0 && tile_cells(h->storage, model, (long long)h->nx * h->ny);
 }
 
-int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
-                bool as_single) {
+static StepArgs tile_args(const plbm_lattice *h, const void *src, void *dst, void *lag) {
     StepArgs a{};
     a.src = src;
     a.dst = dst;
@@ -96,6 +95,12 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
     a.lambda_odd_f = float(h->lambda_odd);
     a.scale = float(h->scale);
     a.inv_scale = float(1.0 / h->scale);
+    return a;
+}
+
+int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
+                bool as_single) {
+    StepArgs a = tile_args(h, src, dst, lag);
     a.round_levels = as_single && h->storage == PLBM_F16S;
     int shape = 0, wx, wy;
     pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
@@ -119,6 +124,31 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
                 return PLBM_OK;
             });
         });
+    });
+}
+
+int launch_tile_levels(plbm_lattice *h, int ns, const void *src, void *dst) {
+    StepArgs a = tile_args(h, src, dst, nullptr);
+    a.level_stride = h->elems;
+    int shape = 0, wx, wy;
+    pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
+    tile_limits(shape, ns, &wx, &wy);
+    const int nbx = (h->nx + wx - 1) / wx, nby = (h->ny + wy - 1) / wy;
+    return dispatch_storage(h->storage, [&](auto S) {
+        constexpr int SS = decltype(S)::value;
+        if constexpr (SS == PLBM_F16S) {
+            set_error("passes that keep every level need FP64 or FP32 storage");
+            return PLBM_ERR_ARG;
+        } else {
+            return dispatch_tile_shape(shape, [&](auto sh) {
+                using SH = decltype(sh);
+                hipLaunchKernelGGL((k_tile<PLBM_BGK, SS, SH, false, true>),
+                                   dim3((unsigned)(nbx * nby)), dim3(SH::T), 0, h->stream, a, ns,
+                                   nbx, nby);
+                PLBM_HIP(hipGetLastError());
+                return PLBM_OK;
+            });
+        }
     });
 }
 

@@ -77,7 +77,10 @@ static_assert(opposite(1) == 3 && opposite(2) == 4 && opposite(3) == 1 && opposi
                   opposite(5) == 7 && opposite(6) == 8 && opposite(7) == 5 && opposite(8) == 6,
               "opposite directions");
 
+// v modulo n; the division only where v is more than one period off.
 __device__ __forceinline__ int wrap_index(int v, int n) {
+    v += v < 0 ? n : 0;
+    v -= v >= n ? n : 0;
     if (v < 0 || v >= n) {
         v %= n;
         if (v < 0) v += n;
@@ -112,6 +115,7 @@ constexpr bool tile_wide(int storage, int model) {
 // The calling workgroup (SHAPE::T threads) advances cells [x0, x0 + w) x [y0, y0 + h) of
 // the grid described by `a` ns >= 1 steps, a.src -> a.dst, and, when a.lag is set (ns >= 2),
 // stores the state one step before there.  w + 2 (ns - 1) <= XW, h + 2 (ns - 1) <= H.
+// KEEP: every level is stored (StepArgs::level_stride).
 //
 // LDS holds one copy of the region's populations, updated in place.  A step pulls f_q(x)
 // from cell x - c_q, so writing the result where it was read from (A: the value of the
@@ -120,7 +124,7 @@ constexpr bool tile_wide(int storage, int model) {
 // written back to (x, p)).  Every LDS word is read and written by the same thread in a
 // step, so that one barrier per step suffices, any number of cells per thread works, and
 // half the LDS of a ping-pong pair holds the tile.
-template <int MODEL, int ST, class SHAPE, bool WIDE = false>
+template <int MODEL, int ST, class SHAPE, bool WIDE = false, bool KEEP = false>
 __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, int w, int y0,
                                            int h) {
     using T = typename Traits<ST>::T;
@@ -179,7 +183,8 @@ __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, in
             R *m = mem + lx * 9 * H + ly;
 #pragma unroll
             for (int q = 0; q < 9; ++q) m[q * H] = f[q];
-            if (halo == 1 && lag != nullptr) store(lag, lx, ly, f);
+            if constexpr (KEEP) store(d, lx, ly, f);
+            else if (halo == 1 && lag != nullptr) store(lag, lx, ly, f);
         }
     }
     // levels 2 .. ns, each one cell smaller on every side: the even ones A, the odd ones B
@@ -197,14 +202,15 @@ __device__ __forceinline__ void tile_steps(const StepArgs &a, int ns, int x0, in
                 f[q] = ODD ? m[opposite(q) * H] : m[(q - 9 * cx(q)) * H - cy(q)];
             collide_tile<MODEL, ST, WIDE>(f, a);
             if constexpr (LAST) {
-                store(d, lx, ly, f);
+                store(KEEP ? d + (size_t)(k - 1) * a.level_stride : d, lx, ly, f);
             } else {
                 settle(f);
 #pragma unroll
                 for (int q = 0; q < 9; ++q)
                     if constexpr (ODD) m[q * H] = f[q];
                     else m[(q - 9 * cx(q)) * H - cy(q)] = f[opposite(q)];
-                if (k == halo && lag != nullptr) store(lag, lx, ly, f);
+                if constexpr (KEEP) store(d + (size_t)(k - 1) * a.level_stride, lx, ly, f);
+                else if (k == halo && lag != nullptr) store(lag, lx, ly, f);
             }
         }
     };
