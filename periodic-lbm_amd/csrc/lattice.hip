@@ -391,6 +391,15 @@ int launch_step(plbm_lattice *h, int model, const void *src, void *dst) {
     return launch_step_cfg(h, model, src, dst, h->cfg[model]);
 }
 
+// Threads per workgroup of the single-step kernel until the caller sets or tunes them: 128 on
+// columns of up to 1024 cells that 256 pad by more, else 256.  us per step, 128 / 256: 320^2
+// BGK 4.0 / 4.8, RR 4.4 / 5.0, FP32 3.2 / 3.5 (RR 3.2 / 3.8), FP16 2.9 / 3.1; 700 x 300 BGK
+// 6.1 / 7.0, RR 6.3 / 7.3; where the padding is the same 256 is as fast or faster (256^2 RR 3.9
+// / 3.8, 400^2 RR 6.2 / 5.9, 1000^2 FP32 16.0 / 15.7, 8192^2 FP32 800 / 769).
+static int default_block(int ny) {
+    return ny <= 1024 && (ny + 127) / 128 * 128 < (ny + 255) / 256 * 256 ? 128 : 256;
+}
+
 static bool valid_cfg(LaunchCfg c) {
     return c.block >= 64 && c.block <= 1024 && c.block % 64 == 0 && (c.remap == 0 || c.remap == 1);
 }
@@ -566,6 +575,7 @@ int plbm_create(int nx, int ny, int nf, int storage, plbm_lattice **out) try {
     h->storage = storage;
     h->elems = (size_t)9 * nx * ldd;
     h->scale = storage == PLBM_F16S ? 1024.0 : 1.0;
+    for (LaunchCfg &c : h->cfg) c.block = default_block(ny);
     if (hipGetDevice(&h->device) != hipSuccess ||
         hipStreamCreateWithFlags(&h->own, hipStreamNonBlocking) != hipSuccess) {
         (void)hipGetLastError();

@@ -86,3 +86,25 @@ def test_automatic_depth_under_capture(P, gpu):
         ref.run("trt", steps, 0, 1)
         for b in (0, 1):
             np.testing.assert_array_equal(lat.download_f(b), ref.download_f(b), err_msg=str(replay))
+
+
+@pytest.mark.parametrize("storage", ["f64", "f16s"])
+@pytest.mark.parametrize("ny,block", [(1, 128), (127, 128), (128, 128), (129, 256), (256, 256),
+                                      (257, 128), (384, 128), (385, 256), (1024, 256),
+                                      (1025, 256)])
+def test_single_step_workgroups(P, gpu, ny, block, storage):
+    """Automatic workgroup sizes of single steps against 256 threads, bit for bit."""
+    print(f"case single steps 7x{ny} {storage}", flush=True)
+    rng = np.random.default_rng(ny)
+    m = [c + 0.02 * rng.standard_normal((ny, 7)) for c in (1.0, 0.0, 0.0)]
+    f = []
+    for chosen in (None, 256):
+        lat = P.Lattice(7, ny, 2, storage)
+        lat.set_params(1.7, 0.25)
+        assert lat.get_launch("rr") == (block, 1)
+        if chosen:
+            lat.set_launch("rr", chosen)
+        lat.equilibrium_init(0, *m)
+        lat.step("rr", 0, 1)
+        f.append(lat.download_f(1)[:ny])
+    np.testing.assert_array_equal(f[0], f[1])
