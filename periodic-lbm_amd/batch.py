@@ -116,7 +116,7 @@ class Batch:
 
     def macros(self, c):
         nx, ny = self.sizes[c]
-        r, u, v = (np.zeros((ny, nx), order="F") for _ in range(3))
+        r, u, v = (np.empty((ny, nx), order="F") for _ in range(3))
         check(lib().plbm_batch_macros(self.h, c, dptr(r), dptr(u), dptr(v)))
         return r, u, v
 

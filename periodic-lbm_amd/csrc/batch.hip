@@ -314,6 +314,7 @@ struct plbm_batch {
     // cached graphs: key = (nsteps, parity at start)
     std::map<std::pair<int, int>, hipGraphExec_t> graphs;
     double *d_red = nullptr;
+    HostStage stage;  // read-back of small fields
     double *d_tmp = nullptr;
     size_t tmp_bytes = 0;
 };
@@ -686,6 +687,7 @@ int plbm_batch_destroy(plbm_batch *b) try {
     if (b->d_cases) (void)hipFree(b->d_cases);
     if (b->d_red) (void)hipFree(b->d_red);
     if (b->d_tmp) (void)hipFree(b->d_tmp);
+    b->stage.release();
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
     if (b->side) (void)hipStreamDestroy(b->side);
@@ -810,16 +812,22 @@ int plbm_batch_macros(plbm_batch *b, int c, double *rho, double *ux, double *uy)
     PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
     const BatchCase &k = b->cases[c];
     const size_t n = (size_t)k.nx * k.ny;
-    PLBM_TRY(ensure_btmp(b, 3 * n * sizeof(double)));
-    const void *src = static_cast<const char *>(b->arena) +
+    const char *src = static_cast<const char *>(b->arena) +
                       (k.off + (b->parity ? k.elems : 0)) * storage_bytes(b->storage);
-    PLBM_TRY(dispatch_storage(b->storage, [&](auto S) {
-        hipLaunchKernelGGL(k_batch_macros<decltype(S)::value>, dim3((k.ny + 255) / 256, k.nx),
-                           dim3(256), 0, b->stream, src, b->d_tmp, b->d_tmp + n, b->d_tmp + 2 * n,
-                           k.nx, k.ny, k.ldd, float(1.0 / b->scale));
-        PLBM_HIP(hipGetLastError());
-        return PLBM_OK;
-    }));
+    auto launch = [&](size_t x0, size_t cols, double *r, double *u, double *v) {
+        const void *from = src + x0 * 9 * k.ldd * storage_bytes(b->storage);
+        return dispatch_storage(b->storage, [&](auto S) {
+            hipLaunchKernelGGL(k_batch_macros<decltype(S)::value>,
+                               dim3((k.ny + 255) / 256, (unsigned)cols), dim3(256), 0, b->stream,
+                               from, r, u, v, (int)cols, k.ny, k.ldd, float(1.0 / b->scale));
+            PLBM_HIP(hipGetLastError());
+            return PLBM_OK;
+        });
+    };
+    if (b->stage.ready(3 * n * sizeof(double)))
+        return fields_through_stage(b->stage, b->stream, k.nx, k.ny, launch, rho, ux, uy);
+    PLBM_TRY(ensure_btmp(b, 3 * n * sizeof(double)));
+    PLBM_TRY(launch(0, (size_t)k.nx, b->d_tmp, b->d_tmp + n, b->d_tmp + 2 * n));
     PLBM_HIP(hipMemcpyAsync(rho, b->d_tmp, n * 8, hipMemcpyDeviceToHost, b->stream));
     PLBM_HIP(hipMemcpyAsync(ux, b->d_tmp + n, n * 8, hipMemcpyDeviceToHost, b->stream));
     PLBM_HIP(hipMemcpyAsync(uy, b->d_tmp + 2 * n, n * 8, hipMemcpyDeviceToHost, b->stream));

@@ -204,6 +204,59 @@ inline int plane_from_host(double *dev, const double *host, size_t ld, size_t ny
     return PLBM_OK;
 }
 
+// Pinned memory through which small fields reach the caller's pageable arrays: a kernel stores
+// them there over the bus, in two halves so that one half's copy on the host overlaps the
+// other's transfer.  Kept by its lattice or batch.  Reading three fields back took, by three
+// copies into pageable memory, at 64^2 / 128^2 / 200^2 / 256^2 / 320^2, 81 / 59 / 83 / 108 / 146
+// us; this 30 / 40 / 60 / 80 / 110.  Larger fields keep the copies, which fault fresh pages in
+// in bulk (512^2 450 us, against 3.6 ms of page faults in a copy on the host).  1 MiB takes 45
+// us to allocate, the most, 2.5 MiB, 280: hence two sizes.
+struct HostStage {
+    void *mem = nullptr;
+    size_t bytes = 0;
+    hipEvent_t half = nullptr;
+    bool failed = false;
+    bool ready(size_t need) {
+        const size_t small = (size_t)1 << 20, most = (size_t)5 << 19;
+        if (need > most || failed) return false;
+        if (bytes >= need) return true;
+        release();
+        bytes = need > small ? most : small;
+        if (hipHostMalloc(&mem, bytes, hipHostMallocDefault) != hipSuccess ||
+            hipEventCreateWithFlags(&half, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            failed = true;
+        }
+        return !failed;
+    }
+    void release() {
+        if (half) (void)hipEventDestroy(half);
+        if (mem) (void)hipHostFree(mem);
+        mem = nullptr;
+        bytes = 0;
+        half = nullptr;
+    }
+};
+
+// Three fields of nx columns of ny into host arrays; launch(x0, columns, rho, ux, uy) issues
+// the kernel for some columns on s.
+template <class F>
+inline int fields_through_stage(HostStage &st, hipStream_t s, size_t nx, size_t ny, F &&launch,
+                                double *rho, double *ux, double *uy) {
+    double *m = static_cast<double *>(st.mem);
+    const size_t x1 = nx / 2, n = nx * ny, n1 = x1 * ny;
+    if (x1 > 0) PLBM_TRY(launch((size_t)0, x1, m, m + n, m + 2 * n));
+    PLBM_HIP(hipEventRecord(st.half, s));
+    PLBM_TRY(launch(x1, nx - x1, m + n1, m + n + n1, m + 2 * n + n1));
+    double *const out[3] = {rho, ux, uy};
+    PLBM_HIP(hipEventSynchronize(st.half));
+    for (int c = 0; c < 3; ++c) std::copy(m + c * n, m + c * n + n1, out[c]);
+    PLBM_HIP(hipStreamSynchronize(s));
+    for (int c = 0; c < 3; ++c) std::copy(m + c * n + n1, m + (c + 1) * n, out[c] + n1);
+    return PLBM_OK;
+}
+
 }  // namespace plbm
 
 struct plbm_lattice;
@@ -261,6 +314,7 @@ struct plbm_lattice {
     std::vector<hipEvent_t> run_events;
     std::vector<int> run_depths;
     // scratch (allocated on first use)
+    plbm::HostStage stage;         // read-back of small fields
     double *d_tmp = nullptr;       // staging for host transfers
     size_t tmp_bytes = 0;
     double *d_partials = nullptr;  // kReduceBlocks * PLBM_NRED

@@ -606,6 +606,7 @@ int plbm_destroy(plbm_lattice *h) try {
     for (int b = 0; b < kMaxBuffers; ++b)
         if (h->f[b]) (void)hipFree(h->f[b]);
     if (h->aux) (void)hipFree(h->aux);
+    h->stage.release();
     for (hipEvent_t e : h->run_events) (void)hipEventDestroy(e);
     if (h->d_tmp) (void)hipFree(h->d_tmp);
     if (h->d_partials) (void)hipFree(h->d_partials);
@@ -824,16 +825,23 @@ int plbm_copy(plbm_lattice *h, int src, int dst) try {
     return plbm::host_exception();
 }
 
-int plbm_macros_dev(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) try {
-    PLBM_TRY(check_buf(h, buf));
-    PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
+static int launch_macros(plbm_lattice *h, int buf, size_t x0, size_t cols, double *rho,
+                         double *ux, double *uy) {
     return dispatch_storage(h->storage, [&](auto S) {
-        hipLaunchKernelGGL(k_macros<decltype(S)::value>, cell_grid(h), dim3(256), 0, h->stream,
-                           h->f[buf], h->nx, h->ny, h->ldd, float(1.0 / h->scale), rho,
-                           ux, uy);
+        constexpr int SS = decltype(S)::value;
+        const auto *src = static_cast<const typename Traits<SS>::T *>(h->f[buf]);
+        hipLaunchKernelGGL(k_macros<SS>, dim3((unsigned)((h->ny + 255) / 256), (unsigned)cols),
+                           dim3(256), 0, h->stream, src + x0 * 9 * h->ldd, (int)cols, h->ny,
+                           h->ldd, float(1.0 / h->scale), rho, ux, uy);
         PLBM_HIP(hipGetLastError());
         return PLBM_OK;
     });
+}
+
+int plbm_macros_dev(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) try {
+    PLBM_TRY(check_buf(h, buf));
+    PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
+    return launch_macros(h, buf, 0, (size_t)h->nx, rho, ux, uy);
 } catch (...) {
     return plbm::host_exception();
 }
@@ -842,8 +850,15 @@ int plbm_macros(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) t
     PLBM_TRY(check_buf(h, buf));
     PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
     const size_t n = (size_t)h->nx * h->ny;
+    if (h->stage.ready(3 * n * sizeof(double)))
+        return fields_through_stage(
+            h->stage, h->stream, h->nx, h->ny,
+            [&](size_t x0, size_t cols, double *r, double *u, double *v) {
+                return launch_macros(h, buf, x0, cols, r, u, v);
+            },
+            rho, ux, uy);
     PLBM_TRY(ensure_tmp(h, 3 * n * sizeof(double)));
-    PLBM_TRY(plbm_macros_dev(h, buf, h->d_tmp, h->d_tmp + n, h->d_tmp + 2 * n));
+    PLBM_TRY(launch_macros(h, buf, 0, (size_t)h->nx, h->d_tmp, h->d_tmp + n, h->d_tmp + 2 * n));
     PLBM_HIP(hipMemcpyAsync(rho, h->d_tmp, n * 8, hipMemcpyDeviceToHost, h->stream));
     PLBM_HIP(hipMemcpyAsync(ux, h->d_tmp + n, n * 8, hipMemcpyDeviceToHost, h->stream));
     PLBM_HIP(hipMemcpyAsync(uy, h->d_tmp + 2 * n, n * 8, hipMemcpyDeviceToHost, h->stream));

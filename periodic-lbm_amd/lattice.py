@@ -256,7 +256,7 @@ class Lattice:
 
     # --- read-back
     def macros(self, buf: int):
-        rho, ux, uy = (np.zeros((self.ny, self.nx), order="F") for _ in range(3))
+        rho, ux, uy = (np.empty((self.ny, self.nx), order="F") for _ in range(3))
         check(lib().plbm_macros(self.h, buf, dptr(rho), dptr(ux), dptr(uy)))
         return rho, ux, uy
 
@@ -644,8 +644,13 @@ def update_macros(grid: LatticeGrid) -> None:
     """update_macros (src/fvm_bardow.F90:343-390): rho, u of f(inew) into grid.mf."""
     if grid._host_current:
         sync_device(grid)
-    rho, ux, uy = grid.lattice.macros(grid.inew - 1)
-    grid.mf[:, :, 0], grid.mf[:, :, 1], grid.mf[:, :, 2] = rho, ux, uy
+    lat, mf = grid.lattice, grid.mf
+    planes = [mf[:, :, c] for c in range(3)]
+    if all(p.dtype == np.float64 and p.flags.f_contiguous and p.flags.writeable
+           and p.shape == (lat.ny, lat.nx) for p in planes):  # as alloc_grid makes them
+        check(lib().plbm_macros(lat.h, grid.inew - 1, *map(dptr, planes)))
+    else:
+        mf[:, :, 0], mf[:, :, 1], mf[:, :, 2] = lat.macros(grid.inew - 1)
 
 
 def equilibrium(rho: float, ux: float, uy: float) -> np.ndarray:
