@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4
     const int y0 = part_start(a.ny, nby, by), h = part_start(a.ny, nby, by + 1) - y0;
     const int nx = a.nx, ny = a.ny, halo = ns - 1;
     const size_t L = (size_t)a.ldd;
-    const uint32_t cs = (uint32_t)(a.cs * sizeof(T));  // bytes of a column
+    const Offset cs = (Offset)(a.cs * sizeof(T));  // bytes of a column
     // Cell i of level k: in the tile's region, and its offsets and its neighbours' in a state.
     struct Cell {
         int lx, ly;
@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4
         c.lx = ix + k - 1;
         c.ly = i - ix * hk + k - 1;
         const int x = wrap_index(x0 + c.lx - halo, nx), y = wrap_index(y0 + c.ly - halo, ny);
-        c.c0 = FAR ? (Offset)x * cs : (Offset)__umul24(x, cs);
+        c.c0 = FAR ? (Offset)x * cs : (Offset)__umul24(x, (uint32_t)cs);
         c.r0 = (Offset)y * sizeof(T);
         const Offset xe = (Offset)(nx - 1) * cs, ye = (Offset)(ny - 1) * sizeof(T);
         c.cm = x == 0 ? c.c0 + xe : c.c0 - cs;
