@@ -398,10 +398,13 @@ static void *state(plbm_adjoint *a, int k, int j) {
     return j == 0 ? ckpt(a, k) : static_cast<char *>(a->segment) + (size_t)(j - 1) * a->buf_bytes;
 }
 
+// The adjoint state is FP64 for every storage.
+constexpr TileKind kAdjTiles{sizeof(double), PLBM_BGK};
+
 // Depth of the object's passes.
 static int adj_depth(const plbm_adjoint *a) {
     int shape, ns = 1;
-    pick_tile(a->nx, a->ny, 1, kMaxStepsPerLaunch, &shape, &ns);
+    pick_tile(a->nx, a->ny, kAdjTiles, 1, kMaxStepsPerLaunch, &shape, &ns);
     return ns;
 }
 // f^{n0+1} .. f^{n0+len} of segment k from its checkpoint.
@@ -417,7 +420,7 @@ static int fill_segment(plbm_adjoint *a, int k, int len) {
 // Tiles of a reverse pass of ns steps: shape, columns and rows of the grid of them.
 static void adj_tiles(const plbm_adjoint *a, int ns, int *shape, int *nbx, int *nby) {
     int wx, wy;
-    pick_tile(a->nx, a->ny, ns, ns, shape, &ns);
+    pick_tile(a->nx, a->ny, kAdjTiles, ns, ns, shape, &ns);
     tile_limits(*shape, ns, &wx, &wy);
     *nbx = (a->nx + wx - 1) / wx;
     *nby = (a->ny + wy - 1) / wy;

@@ -339,25 +339,36 @@ static bool batch_tile_cells(int storage, int model, long long cells) {
 }
 
 // LDS tile shape of the passes of a plan, or -1 for column walks (larger batches, or the
-// caller set the walk's columns): the shape whose tiles cost the busiest CU the least.
+// caller set the walk's columns): the shape whose tiles cost the busiest CU the least.  Beyond
+// one tile per CU only the last two shapes are of use, and more of their loads and stores
+// overlap another tile's steps (0.8 and 1.4 steps a cell).  With pick_tile's costs there
+// instead: TRT FP64 5.9 -> 6.9 us per step at 0.7 M cells, RR FP32 4.9 -> 5.2.
 static int pass_shape(const plbm_batch *b, const BatchCfg &cfg) {
     if (cfg.ns < 2 || cfg.walk || tile_wide(b->storage, b->model)) return -1;
     long long cells = 0;
     for (const BatchCase &k : b->cases)
         if ((long long)k.nx * k.ny > cfg.resident_cells) cells += (long long)k.nx * k.ny;
     if (!batch_tile_cells(b->storage, b->model, cells)) return -1;
+    const TileKind kind{(int)storage_bytes(b->storage), b->model};
     int best = -1;
     double cost = 1e300;
     for (int s = 0; s < kTileShapes; ++s) {
         int wx, wy;
         tile_limits(s, cfg.ns, &wx, &wy);
-        double work = 0, n = 0;
+        double work = 0, crowded = 0, n = 0;
         for (const BatchCase &k : b->cases) {
             if ((long long)k.nx * k.ny <= cfg.resident_cells) continue;
             const int nbx = (k.nx + wx - 1) / wx, nby = (k.ny + wy - 1) / wy;
+            const int w = (k.nx + nbx - 1) / nbx, h = (k.ny + nby - 1) / nby;
             const double m = double(nbx) * nby;
             n += m;
-            work += m * tile_work(s, cfg.ns, (k.nx + nbx - 1) / nbx, (k.ny + nby - 1) / nby);
+            work += m * tile_work(s, kind, cfg.ns, w, h);
+            crowded += m * (tile_cell_steps(cfg.ns, w, h) +
+                            (s == kTileM ? 0.8 : 1.4) * tile_cells_moved(cfg.ns, w, h));
+        }
+        if (n > kComputeUnits) {
+            if (s < kTileM) continue;
+            work = crowded;
         }
         const double c = n > 0 ? std::ceil(n / kComputeUnits) * work / n : 0;
         if (c < cost) {

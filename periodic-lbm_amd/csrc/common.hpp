@@ -277,7 +277,12 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
 // One pass of ns >= 1 BGK steps that stores every level (F64, F64S, F32S storage), the roundings
 // of single steps: level k into the k-th of ns consecutive buffers at dst.
 int launch_tile_levels(plbm_lattice *h, int ns, const void *src, void *dst);
-double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
+// What the choice of a tile's shape and depth depends on beside the grid.
+struct TileKind {
+    int bytes, model;  // of a stored value; the collision
+};
+TileKind tile_kind(const plbm_lattice *h, int model);
+double pick_tile(int nx, int ny, TileKind kind, int ns_min, int ns_max, int *shape, int *ns);
 // Run bookkeeping shared by the pass runs (multistep.hip): pass depths of a run, the
 // lattice's third buffer (nullptr when it cannot be allocated), and the final assignment
 // of device storage to slots.

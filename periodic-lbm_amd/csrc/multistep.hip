@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "multistep.hpp"
+#include "tile.hpp"
 
 namespace plbm {
 
@@ -111,7 +112,7 @@ int default_steps_per_launch(const plbm_lattice *h, int model) {
 
 int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
                  void *lag, bool as_single) {
-    if (ns >= 2 && ns <= kMaxPassSteps && tile_grid(h, model))
+    if (ns >= 2 && ns <= kMaxTileSteps && tile_grid(h, model))
         return launch_tile(h, model, ns, src, dst, lag, as_single);
     StepArgs a{};
     a.src = src;
@@ -270,7 +271,7 @@ static int timing_mark(plbm_lattice *h, int depth) {
 
 //
 // A grid that takes tiles chooses the depth itself when the caller has not
-// (plbm_set_steps_per_launch): the cheapest of 2..8 (pick_tile), spread evenly over the
+// (plbm_set_steps_per_launch): the cheapest of 2..11 (tile_depth), spread evenly over the
 // passes.  On grids of fewer than 512 column walks the passes stand for single steps and
 // round as they do (as_single).  On larger ones FP16 storage, which rounds a state whenever it
 // is stored, keeps the depth of 8.
@@ -279,15 +280,14 @@ static int timing_mark(plbm_lattice *h, int depth) {
 int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
     int ns = h->cfg[model].ns, lag_ns = h->cfg[model].lag_ns;
     bool even = false, as_single = false;
-    if (ns == 0) {
+    if (ns == 0 && nsteps >= 2) {
         const bool walks = enough_walks(h);
         ns = walks ? kMaxPassSteps : 1;
         if (tile_grid(h, model) && (!walks || h->storage != PLBM_F16S)) {
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
             if (!walks) PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
             if (cap == hipStreamCaptureStatusNone) {
-                int shape;
-                pick_tile(h->nx, h->ny, 2, kMaxPassSteps, &shape, &ns);
+                ns = tile_depth(h->nx, h->ny, tile_kind(h, model), nsteps);
                 even = true;
                 as_single = !walks;
             }

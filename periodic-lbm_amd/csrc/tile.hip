@@ -12,10 +12,12 @@
 // cells per thread and iteration, to overlap one's LDS reads with the other's collision,
 // measured 3-20% slower.
 //
-// us per step, single steps / column walk of 8 / tiles: 64^2 BGK FP64 3.4 / 5.5 / 1.1;
+// us per step, single steps / column walk of 8 / tiles: 64^2 BGK FP64 3.4 / 5.5 / 0.9;
 // 192^2 TRT FP64 3.6 / 4.9 / 1.2; 512^2 TRT FP64 8.3 / 5.0 / 2.3, FP32 4.3 / 3.5 / 1.6;
 // 1001 x 777 RR FP64 23.8 / 24.5 / 10.1; 1024^2 TRT FP64 29 / 10.0 / 8.4, FP32 16.4 / 5.8 /
-// 4.2.
+// 4.2.  Tiles of up to 11 steps in four shapes instead of up to 8 in three, 512^2 and larger
+// ones mostly the same: 64^2 BGK FP64 1.08 -> 0.90, 128^2 TRT FP64 1.15 -> 0.97, 320^2 RR
+// FP64 2.43 -> 2.23, 400^2 TRT FP64 2.50 -> 1.99, 640^2 TRT FP64 5.3 -> 4.1, FP32 3.1 -> 2.1.
 //
 // Per-cell arithmetic is collide_cell, as everywhere: FP64 results equal single steps bit
 // for bit, and the shifted FP64 / FP32 storages did on every case compared (but see
@@ -34,7 +36,7 @@ __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4
     tile_steps<MODEL, ST, SHAPE, WIDE, KEEP>(a, ns, x0, x1 - x0, y0, y1 - y0);
 }
 
-double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
+double pick_tile(int nx, int ny, TileKind kind, int ns_min, int ns_max, int *shape, int *ns) {
     double best = 1e300;
     for (int n = ns_min; n <= ns_max; ++n)
         for (int s = 0; s < kTileShapes; ++s) {
@@ -44,7 +46,8 @@ double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
             w = (int)((nx + nbx - 1) / nbx);
             h = (int)((ny + nby - 1) / nby);
             const double per_cu = double((nbx * nby + kComputeUnits - 1) / kComputeUnits);
-            const double c = (kTileLaunchWork + per_cu * tile_work(s, n, w, h)) / n;
+            const double c =
+                (tile_launch_work(kind) + per_cu * tile_work(s, kind, n, w, h)) / n;
             if (c < best) {
                 best = c;
                 *shape = s;
@@ -52,6 +55,26 @@ double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns) {
             }
         }
     return best;
+}
+
+int tile_depth(int nx, int ny, TileKind kind, int nsteps) {
+    double cost[kMaxTileSteps + 1] = {}, least = 1e300;
+    int best = 2;
+    for (int n = 1; n <= kMaxTileSteps; ++n) {
+        int shape, ns;
+        cost[n] = n * pick_tile(nx, ny, kind, n, n, &shape, &ns);
+        const int passes = (nsteps + n - 1) / n, d = nsteps / passes, deeper = nsteps % passes;
+        const double c = (passes - deeper) * cost[d] + (deeper ? deeper * cost[d + 1] : 0.0);
+        if (n >= 2 && c < least) {
+            least = c;
+            best = n;
+        }
+    }
+    return best;
+}
+
+TileKind tile_kind(const plbm_lattice *h, int model) {
+    return {(int)storage_bytes(h->storage), model};
 }
 
 // Grids up to this many cells take tiles: about where the column walk catches up.  us per
@@ -103,7 +126,7 @@ int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, 
     StepArgs a = tile_args(h, src, dst, lag);
     a.round_levels = as_single && h->storage == PLBM_F16S;
     int shape = 0, wx, wy;
-    pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
+    pick_tile(h->nx, h->ny, tile_kind(h, model), ns, ns, &shape, &ns);
     tile_limits(shape, ns, &wx, &wy);
     const int nbx = (h->nx + wx - 1) / wx, nby = (h->ny + wy - 1) / wy;
     return dispatch_model(model, [&](auto M) {
@@ -131,7 +154,7 @@ int launch_tile_levels(plbm_lattice *h, int ns, const void *src, void *dst) {
     StepArgs a = tile_args(h, src, dst, nullptr);
     a.level_stride = h->elems;
     int shape = 0, wx, wy;
-    pick_tile(h->nx, h->ny, ns, ns, &shape, &ns);
+    pick_tile(h->nx, h->ny, tile_kind(h, PLBM_BGK), ns, ns, &shape, &ns);
     tile_limits(shape, ns, &wx, &wy);
     const int nbx = (h->nx + wx - 1) / wx, nby = (h->ny + wy - 1) / wy;
     return dispatch_storage(h->storage, [&](auto S) {

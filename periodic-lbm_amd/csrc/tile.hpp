@@ -11,27 +11,32 @@
 namespace plbm {
 
 // A tile's region at level 1 holds at most XW columns of H rows; T threads work on it.
-// LDS of the three shapes in FP64: 41, 78 and 159 of a CU's 160 KB, so that 3, 2 and 1
-// workgroups share a CU (16-24 wavefronts either way).  Measured and not kept: S with 256
-// threads (5-15% slower), M with 1024, L with 512 or 768 (3-13% slower), 18 x 18 (slower
-// beyond 64^2), 40 x 36, and 70 x 64 for 4-byte values (5-45% slower than L).
-template <int XW_, int H_, int T_, int MEM_>
+// LDS of the shapes in FP64: 41, 73, 78 and 159 of a CU's 160 KB.  The first two are for grids
+// that give a CU one tile: its 16 wavefronts then take at most one cell per thread and level
+// (64^2 BGK FP64 11 steps, 24 x 24 with 512 / 576 / 1024 threads: 1.00 / 0.95 / 0.95 us per
+// step; 128^2 TRT 9 steps 1.05 / 1.02 / 0.97).  Measured and not kept: 24 x 24 with 256, 320 or
+// 512 threads (5-15% slower, or within 4%), M with 1024, L with 512 or 768 (3-13% slower),
+// 18 x 18, 40 x 36, and 70 x 64 for 4-byte values (5-45% slower than L).
+template <int XW_, int H_, int T_, int MEM8_, int MEM4_ = MEM8_>
 struct TileShape {
     static constexpr int XW = XW_, H = H_, T = T_;
-    // cost of moving one cell between memory and LDS, in tenths of a cell's step: the
-    // more workgroups share a CU, the more of it overlaps another's steps
-    static constexpr int MEM = MEM_;
+    // cost of moving one cell between memory and LDS, in hundredths of a cell's step, for
+    // 8-byte values and for smaller ones (see pick_tile)
+    static constexpr int MEM8 = MEM8_, MEM4 = MEM4_;
 };
-using TileS = TileShape<24, 24, 512, 7>;
-using TileM = TileShape<34, 32, 512, 8>;
-using TileL = TileShape<48, 46, 1024, 14>;
-constexpr int kTileShapes = 3;
+using TileS = TileShape<24, 24, 1024, 80>;
+using TileW = TileShape<32, 32, 1024, 125>;
+using TileM = TileShape<34, 32, 512, 100, 300>;
+using TileL = TileShape<48, 46, 1024, 155>;
+constexpr int kTileShapes = 4, kTileM = 2;  // S, W, M, L
+constexpr int kMaxTileSteps = 11;  // leaves S tiles of 4 x 4
 
 template <class F>
 inline int dispatch_tile_shape(int shape, F &&f) {
     switch (shape) {
     case 0: return f(TileS{});
-    case 1: return f(TileM{});
+    case 1: return f(TileW{});
+    case kTileM: return f(TileM{});
     default: return f(TileL{});
     }
 }
@@ -46,24 +51,41 @@ inline void tile_limits(int shape, int ns, int *w, int *h) {
     });
 }
 
-// Work of one tile of w x h cells and ns steps, in steps of a cell: the steps of its
-// shrinking levels, and the load of its region and the store of its cells.
-inline double tile_work(int shape, int ns, int w, int h) {
+// Work of one tile of w x h cells and ns steps, in steps of a BGK or TRT cell: the steps of
+// its shrinking levels, the load of its region and the store of its cells, and a ramp of 300.
+// In RR steps, 1.45 times as long, the latter two are the less.
+inline double tile_heavy(TileKind kind) { return kind.model == PLBM_RR ? 1.45 : 1.0; }
+inline double tile_cell_steps(int ns, int w, int h) {
     double c = 0;
     for (int k = 0; k < ns; ++k) c += double(w + 2 * k) * (h + 2 * k);
-    dispatch_tile_shape(shape, [&](auto s) {
-        c += 0.1 * decltype(s)::MEM * (double(w + 2 * ns) * (h + 2 * ns) + double(w) * h);
-        return 0;
-    });
     return c;
 }
-constexpr double kTileLaunchWork = 2500;  // a launch and its ramp, in the same unit
+inline double tile_cells_moved(int ns, int w, int h) {
+    return double(w + 2 * ns) * (h + 2 * ns) + double(w) * h;
+}
+inline double tile_work(int shape, TileKind kind, int ns, int w, int h) {
+    const int mem = dispatch_tile_shape(shape, [&](auto s) {
+        return kind.bytes == 8 ? decltype(s)::MEM8 : decltype(s)::MEM4;
+    });
+    return tile_cell_steps(ns, w, h) +
+           (0.01 * mem * tile_cells_moved(ns, w, h) + 300) / tile_heavy(kind);
+}
+// A launch and its ramp, in the same unit (TRT FP64: 0.9 ns).
+inline double tile_launch_work(TileKind kind) {
+    return (kind.bytes == 8 ? 3000 : 4400) / tile_heavy(kind);
+}
 
 // The shape and depth (in [ns_min, ns_max]) that cost the least per step on an nx x ny
-// grid; returns the cost of a step.  The busiest CU sets the time: ceil(tiles / 256) tiles
-// of the work above (TRT FP64: 0.9 ns a unit).  Over 32^2 to 2048^2, four collisions and
-// three storages the choice is within 8% of the fastest measured shape and depth.
-double pick_tile(int nx, int ny, int ns_min, int ns_max, int *shape, int *ns);
+// grid; returns the cost of a step.  The busiest CU sets the time: ceil(tiles / 256) tiles of
+// the work above.  Its constants are fitted to every shape and depth to 16 on 16 grids of
+// 32^2 to 1280^2, three collisions each: the choice is on average 0.3% (FP64) and 0.7% (FP32)
+// slower than the fastest measured, at most 4% and 18%.  The depth that leaves just 256 tiles
+// mostly wins, e.g. TRT FP64 640^2 4 steps of L, 5.3 -> 4.1 us per step, 400^2 11 steps of L,
+// 2.5 -> 2.0.
+double pick_tile(int nx, int ny, TileKind kind, int ns_min, int ns_max, int *shape, int *ns);
+
+// The depth that makes nsteps >= 2 steps, spread evenly over their passes, cost the least.
+int tile_depth(int nx, int ny, TileKind kind, int nsteps);
 
 // Column / row boundary j of n cells cut into m nearly equal parts, long and short ones mixed
 // (all longer ones first made the last CUs to finish later: 1001 x 777 RR passes 4%, batches

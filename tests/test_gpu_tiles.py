@@ -64,6 +64,27 @@ def test_automatic_depth_equals_single_steps(P, gpu, storage, model):
         np.testing.assert_array_equal(lat.download_f(n), ref.download_f(n))
 
 
+@pytest.mark.parametrize("model", ["bgk", "trt", "rr"])
+def test_automatic_depths_fp64(P, gpu, oracle, model):
+    """The depths a run chooses, beyond 8 among them, at the edges of the one tile per compute
+    unit that it chooses them for: oracle, bit for bit."""
+    deepest = {}
+    for nx, ny, steps in ((2, 3, 11), (32, 32, 23), (64, 64, 22), (65, 63, 12), (96, 97, 31),
+                          (128, 128, 9), (129, 127, 19), (255, 256, 18), (257, 256, 10),
+                          (320, 320, 7), (321, 319, 8), (400, 400, 11), (401, 399, 13)):
+        print(f"case tile depth {model} {nx}x{ny} {steps} steps", flush=True)
+        lat = lattice(P, "f64", nx, ny)
+        lat.set_run_timing(True)
+        i, n = lat.run(model, steps, 0, 1)
+        deepest[nx, ny] = max(d for d, _ in lat.run_launch_times())
+        fa, fb = po.new_f(nx, ny), po.new_f(nx, ny)
+        oracle.set_pdf_to_equilibrium(nx, ny, *fields(nx, ny, 1), fa)
+        latest, prev = oracle.run(model, nx, ny, fa, fb, steps, OMEGA, 0.25)
+        np.testing.assert_array_equal(lat.download_f(i)[:ny], latest[:ny])
+        np.testing.assert_array_equal(lat.download_f(n)[:ny], prev[:ny])
+    assert deepest[64, 64] == 11 and deepest[2, 3] == 11
+
+
 def test_automatic_depth_under_capture(P, gpu):
     """A captured run on a small grid stays in its two buffers, so that replays continue
     from each other; eager runs before and between do not disturb it."""
