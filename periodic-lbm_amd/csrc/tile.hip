@@ -45,9 +45,9 @@ double pick_tile(int nx, int ny, TileKind kind, int ns_min, int ns_max, int *sha
             const long long nbx = (nx + w - 1) / w, nby = (ny + h - 1) / h;
             w = (int)((nx + nbx - 1) / nbx);
             h = (int)((ny + nby - 1) / nby);
-            const double per_cu = double((nbx * nby + kComputeUnits - 1) / kComputeUnits);
-            const double c =
-                (tile_launch_work(kind) + per_cu * tile_work(s, kind, n, w, h)) / n;
+            const double c = (tile_launch_work(kind) + tile_rounds(s, kind, double(nbx * nby)) *
+                                                           tile_work(s, kind, n, w, h)) /
+                             n;
             if (c < best) {
                 best = c;
                 *shape = s;
@@ -78,24 +78,24 @@ TileKind tile_kind(const plbm_lattice *h, int model) {
 }
 
 // Grids up to this many cells take tiles: about where the column walk catches up.  us per
-// step at both sides' automatic depths, column walk / tiles, FP64 | FP32 | FP16 (whose depth
-// stays 8, see run_steps):
-//   BGK   800^2 8.9/6.8 | 5.2/3.3 | 5.5/4.1;    1200^2 14.7/14.5 | 8.3/6.8 | 7.9/7.5;
-//        1400^2 18.0/21.2 | 10.0/8.7 | 10.1/9.9;  1600^2 22.1/33.5 | 11.7/14.0 | 12.2/12.1
-//   TRT   800^2 6.7/5.8 | 4.5/3.2 | 4.2/3.5;    1000^2 8.7/10.4 | 5.4/6.1 | 5.3/4.4;
-//        1200^2 11.2/13.3 | 7.0/6.5 | 6.7/6.2;  1400^2 13.0/19.9 | 8.3/8.2 | 7.9/8.0
-//   RR   1000^2 16.4/13.6 | 9.1/8.3 | 8.6/6.6;  1400^2 26.2/25.3 | 13.8/11.7 | 13.6/12.3;
-//        1600^2 32.2/36.4 | 16.8/18.8 | 16.3/15.7;  2048^2 50.8/54.5 | 25.1/25.3 | 23.1/24.6
-// FP32 BGK in FP64 arithmetic (collide_tile): 512^2 4.4/2.7, 640^2 4.9/4.6, 800^2 5.3/4.9,
-// 1001 x 777 5.8/6.2, 1000^2 5.9/8.6.
+// step of 96 steps at both sides' automatic depths, column walk / tiles:
+//         FP64                                   FP32                    FP16
+//   BGK   1000^2 10.4/9.2, 1150^2 12.8/12.4,     (below)                 1450^2 8.3/8.1,
+//         1300^2 14.4/16.6                                               1600^2 9.3/9.9
+//   TRT   800^2 6.8/5.8, 900^2 7.4/7.8,          1150^2 5.5/5.2,         1150^2 5.6/5.2,
+//         1150^2 10.3/11.4                       1300^2 6.2/7.1          1300^2 6.4/6.9
+//   RR    1150^2 18.2/16.4, 1300^2 22.5/20.8,    1600^2 14.6/13.0,       1450^2 12.9/12.1,
+//         1450^2 26.1/28.4                       2048^2 21.7/22.4        1800^2 18.1/17.7
+// FP32 BGK in FP64 arithmetic (collide_tile): 640^2 4.9/3.9, 800^2 5.3/4.9, 1001 x 777 5.8/5.2,
+// 1024^2 5.9/6.0.
 bool tile_cells(int storage, int model, long long cells) {
     const int bytes = (int)storage_bytes(storage);
     const auto pick = [&](long long f64, long long f32, long long f16) {
         return cells <= (bytes == 8 ? f64 : bytes == 4 ? f32 : f16);
     };
-    if (model == PLBM_TRT) return pick(850000, 1900000, 1700000);
-    if (model == PLBM_RR) return pick(2100000, 2200000, 2600000);
-    return pick(1400000, 700000, 2400000);
+    if (model == PLBM_TRT) return pick(750000, 1400000, 1400000);
+    if (model == PLBM_RR) return pick(1800000, 3300000, 2600000);
+    return pick(1400000, 850000, 2200000);
 }
 
 // A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.

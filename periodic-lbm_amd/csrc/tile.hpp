@@ -4,6 +4,8 @@
 // the batched engine (batch.hip).  See tile.hip for the scheme.
 #pragma once
 
+#include <cmath>
+
 #include "common.hpp"
 #include "d2q9.hpp"
 #include "stepper.hpp"
@@ -17,17 +19,18 @@ namespace plbm {
 // step; 128^2 TRT 9 steps 1.05 / 1.02 / 0.97).  Measured and not kept: 24 x 24 with 256, 320 or
 // 512 threads (5-15% slower, or within 4%), M with 1024, L with 512 or 768 (3-13% slower),
 // 18 x 18, 40 x 36, and 70 x 64 for 4-byte values (5-45% slower than L).
-template <int XW_, int H_, int T_, int MEM8_, int MEM4_ = MEM8_>
+template <int XW_, int H_, int T_, int MEM8_, int MEM4_, int CROWD8_, int CROWD4_>
 struct TileShape {
     static constexpr int XW = XW_, H = H_, T = T_;
-    // cost of moving one cell between memory and LDS, in hundredths of a cell's step, for
-    // 8-byte values and for smaller ones (see pick_tile)
-    static constexpr int MEM8 = MEM8_, MEM4 = MEM4_;
+    // for pick_tile, 8-byte values and smaller ones: cost of moving one cell between memory and
+    // LDS in hundredths of a cell's step, and a tile's time in hundredths of its time alone
+    // where a CU has several (those of M overlap best)
+    static constexpr int MEM8 = MEM8_, MEM4 = MEM4_, CROWD8 = CROWD8_, CROWD4 = CROWD4_;
 };
-using TileS = TileShape<24, 24, 1024, 80>;
-using TileW = TileShape<32, 32, 1024, 125>;
-using TileM = TileShape<34, 32, 512, 100, 300>;
-using TileL = TileShape<48, 46, 1024, 155>;
+using TileS = TileShape<24, 24, 1024, 107, 120, 114, 119>;
+using TileW = TileShape<32, 32, 1024, 100, 115, 105, 103>;
+using TileM = TileShape<34, 32, 512, 103, 135, 91, 80>;
+using TileL = TileShape<48, 46, 1024, 123, 127, 100, 91>;
 constexpr int kTileShapes = 4, kTileM = 2;  // S, W, M, L
 constexpr int kMaxTileSteps = 11;  // leaves S tiles of 4 x 4
 
@@ -51,10 +54,12 @@ inline void tile_limits(int shape, int ns, int *w, int *h) {
     });
 }
 
-// Work of one tile of w x h cells and ns steps, in steps of a BGK or TRT cell: the steps of
-// its shrinking levels, the load of its region and the store of its cells, and a ramp of 300.
-// In RR steps, 1.45 times as long, the latter two are the less.
-inline double tile_heavy(TileKind kind) { return kind.model == PLBM_RR ? 1.45 : 1.0; }
+// RR steps take this many times a BGK or TRT step: memory and launches cost the fewer of them.
+inline double tile_heavy(TileKind kind) {
+    return kind.model != PLBM_RR ? 1.0 : kind.bytes == 8 ? 1.55 : 1.25;
+}
+// Work of one tile of w x h cells and ns steps, in steps of a cell (TRT FP64: 0.9 ns): the
+// steps of its shrinking levels, the load of its region and the store of its cells, and a ramp.
 inline double tile_cell_steps(int ns, int w, int h) {
     double c = 0;
     for (int k = 0; k < ns; ++k) c += double(w + 2 * k) * (h + 2 * k);
@@ -68,20 +73,27 @@ inline double tile_work(int shape, TileKind kind, int ns, int w, int h) {
         return kind.bytes == 8 ? decltype(s)::MEM8 : decltype(s)::MEM4;
     });
     return tile_cell_steps(ns, w, h) +
-           (0.01 * mem * tile_cells_moved(ns, w, h) + 300) / tile_heavy(kind);
+           (0.01 * mem * tile_cells_moved(ns, w, h) + 850) / tile_heavy(kind);
 }
-// A launch and its ramp, in the same unit (TRT FP64: 0.9 ns).
+// Time of the busiest CU when `tiles` tiles are shared out, in units of one tile's work.
+inline double tile_rounds(int shape, TileKind kind, double tiles) {
+    if (tiles <= kComputeUnits) return 1;
+    const int crowd = dispatch_tile_shape(shape, [&](auto s) {
+        return kind.bytes == 8 ? decltype(s)::CROWD8 : decltype(s)::CROWD4;
+    });
+    return 0.01 * crowd * std::ceil(tiles / kComputeUnits);
+}
+// A launch, in the same unit.
 inline double tile_launch_work(TileKind kind) {
-    return (kind.bytes == 8 ? 3000 : 4400) / tile_heavy(kind);
+    return (kind.bytes == 8 ? 2000 : 3400) / tile_heavy(kind);
 }
 
 // The shape and depth (in [ns_min, ns_max]) that cost the least per step on an nx x ny
-// grid; returns the cost of a step.  The busiest CU sets the time: ceil(tiles / 256) tiles of
-// the work above.  Its constants are fitted to every shape and depth to 16 on 16 grids of
-// 32^2 to 1280^2, three collisions each: the choice is on average 0.3% (FP64) and 0.7% (FP32)
-// slower than the fastest measured, at most 4% and 18%.  The depth that leaves just 256 tiles
-// mostly wins, e.g. TRT FP64 640^2 4 steps of L, 5.3 -> 4.1 us per step, 400^2 11 steps of L,
-// 2.5 -> 2.0.
+// grid; returns the cost of a step.  The constants above are fitted to every shape and depth
+// to 16 on 16 grids of 32^2 to 1280^2 and three collisions: the choice, free or at a given
+// depth, is on average 0.2% slower than the fastest measured, at most 4%.  The depth that
+// leaves just 256 tiles mostly wins, e.g. TRT FP64 640^2 4 steps of L, 5.3 -> 4.1 us per step,
+// 400^2 11 steps of L, 2.5 -> 2.0.
 double pick_tile(int nx, int ny, TileKind kind, int ns_min, int ns_max, int *shape, int *ns);
 
 // The depth that makes nsteps >= 2 steps, spread evenly over their passes, cost the least.
