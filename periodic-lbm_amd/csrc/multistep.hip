@@ -104,8 +104,8 @@ static bool enough_walks(const plbm_lattice *h) {
 }
 
 // Most steps of a launch of plbm_run when the caller has not chosen, as reported: 8 where it
-// runs in tiles (which go to 11, see run_steps), or where the column walk has at least 512 wavefronts; else single steps (wide and
-// flat grids beyond the tiles' limit).
+// runs in tiles (which go to 11, see run_steps), or where the column walk has at least 512
+// wavefronts; else single steps (wide and flat grids beyond the tiles' limit).
 int default_steps_per_launch(const plbm_lattice *h, int model) {
     return enough_walks(h) || tile_grid(h, model) ? kMaxPassSteps : 1;
 }
