@@ -280,7 +280,8 @@ int plbm_get_launch(const plbm_lattice *h, int model, int *block, int *xcd_remap
  * kernel; 2..8 = that many fused steps per launch, in tiles held in LDS on small and medium
  * grids and by wavefronts walking segments of columns on larger ones; 0 = chosen from the
  * grid size: launches of up to 8 steps (of up to 11 in tiles, as many as make the run
- * cheapest; the get variant reports 8), or single steps on wide, flat grids beyond the tiles' limit, and while the lattice's stream is being captured on grids below about
+ * cheapest; the get variant reports 8), or single steps on wide, flat grids beyond the
+ * tiles' limit, and while the lattice's stream is being captured on grids below about
  * 512^2).  In F64 storage the results are bit-identical for every setting;
  * the shifted storages agree to roundoff (their collisions allow FMA contraction, which
  * the compiler places per kernel).  plbm_run keeps the reference's slot contents (latest
