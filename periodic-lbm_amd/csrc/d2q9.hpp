@@ -381,39 +381,6 @@ __device__ inline void collide_bgk_shifted_conserving(R g[9], R omega) {
     for (int q = 0; q < 9; ++q) g[q] = g[q] + omega * (geq[q] - g[q]);
 }
 
-// The same operator for FP16 storage in the form of TRT with equal rates: rho u = j, so that
-// the antisymmetric parts of the equilibrium are linear in j and the symmetric ones need
-// j_a j_b / rho alone, on the diagonals 3 e + 9 xy with e = j.j / rho, xy = j_x j_y / rho.  67
-// instead of 81 instructions in passes bound by them (3000 x 1500, 40 steps 680 -> 602 us).  In
-// FP32 storage it would be nearer FP64 too (150 steps 2.6e-7 instead of 9.3e-7), but the small
-// velocity components of long shear-layer runs would move by 3.5e-5 from what they have been,
-// more than FP32 results may: FP32 storage keeps the form above.
-template <class R>
-__device__ inline void collide_bgk_pairs(R g[9], R omega) {
-#pragma clang fp contract(fast)
-    R drho, jx, jy;
-    moments_shifted(g, drho, jx, jy);
-    const R inv = recip(R(1) + drho);
-    const R ux = jx * inv, uy = jy * inv;
-    const R xx = jx * ux, yy = jy * uy, xy = jx * uy;
-    const R diag = drho + R(3) * (xx + yy);
-    const R os = R(0.5) * omega;
-    const R s57 = os * (g[5] + g[7] - R(T2X2) * (diag + R(9) * xy));
-    const R a57 = os * (g[5] - g[7] - R(3.0 * T2X2) * (jx + jy));
-    const R s86 = os * (g[8] + g[6] - R(T2X2) * (diag - R(9) * xy));
-    const R a86 = os * (g[8] - g[6] - R(3.0 * T2X2) * (jx - jy));
-    const R s24 = os * (g[2] + g[4] - R(T1X2) * (drho - R(1.5) * xx + R(3) * yy));
-    const R s13 = os * (g[1] + g[3] - R(T1X2) * (drho - R(1.5) * yy + R(3) * xx));
-    const R a13 = -(a57 + a86), a24 = a86 - a57;
-    const R o0 = g[0] + R(2) * ((s57 + s86) + (s24 + s13));
-    const R o5 = g[5] - s57 - a57, o7 = g[7] - s57 + a57;
-    const R o8 = g[8] - s86 - a86, o6 = g[6] - s86 + a86;
-    const R o2 = g[2] - s24 - a24, o4 = g[4] - s24 + a24;
-    const R o1 = g[1] - s13 - a13, o3 = g[3] - s13 + a13;
-    g[0] = o0; g[1] = o1; g[2] = o2; g[3] = o3; g[4] = o4;
-    g[5] = o5; g[6] = o6; g[7] = o7; g[8] = o8;
-}
-
 template <class R>
 __device__ inline void collide_trt_shifted_conserving(R g[9], R le, R lo) {
 #pragma clang fp contract(fast)

@@ -55,8 +55,7 @@ __device__ __forceinline__ void collide_cell(typename Traits<ST>::R f[9], const 
         const R om = sizeof(R) == 8 ? R(a.omega) : R(a.omega_f);
         const R lo = sizeof(R) == 8 ? R(a.lambda_odd) : R(a.lambda_odd_f);
         if constexpr (sizeof(R) == 4 && (MODEL == PLBM_BGK || MODEL == PLBM_BGK_SPLIT)) {
-            if constexpr (ST == PLBM_F16S) collide_bgk_pairs<R>(f, om);
-            else collide_bgk_shifted_conserving<R>(f, om);
+            collide_bgk_shifted_conserving<R>(f, om);
         } else if constexpr (sizeof(R) == 4 && MODEL == PLBM_TRT) {
             collide_trt_shifted_conserving<R>(f, om, lo);
         } else if constexpr (sizeof(R) == 4) {
