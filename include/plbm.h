@@ -127,7 +127,11 @@ int plbm_step(plbm_lattice *h, int model, int src, int dst);
  * writes *inew, then swaps them.  Runs in passes of several steps where that is faster
  * (plbm_set_steps_per_launch, plbm_set_pass_lag_buffer); the slot contents afterwards are
  * the reference's, but the slots' device storage may have moved (fetch plbm_buffer_ptr
- * again).  Asynchronous. */
+ * again).  A graph captured from calls on the lattice's stream holds the slots' addresses: from
+ * the first captured call on, runs at automatic depths (plbm_run, plbm_run_op,
+ * plbm_dugks_step) leave the latest state where the graph expects it, by single steps on
+ * small grids and fixed pass depths on larger ones (there runs of an even number of
+ * passes).  Asynchronous. */
 int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew);
 /* Unfused operators for the procedure-pointer slots grid%streaming / grid%collision:
  * lbm_stream (src/periodic_lbm.f90:32-129) src -> dst; collide_* in place on buf. */
@@ -169,8 +173,8 @@ int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *iold, int *
                 double dt);
 /* Pass depth of plbm_run_op: 1 = single fused steps, 2..3 = passes (FP64 storage only),
  * 0 = chosen from the grid size (FP64: passes of up to 6 steps, in LDS tiles on small grids
- * and by column walks on larger ones; single steps on grids of fewer than 2048 walks of 64
- * columns while the lattice's stream is being captured).  The get variant reports the
+ * and by column walks on larger ones; from the first captured call on, see plbm_run, single
+ * steps on grids of fewer than 2048 walks of 64 columns, else 3).  The get variant reports the
  * effective value for (op, model). */
 int plbm_set_op_steps_per_pass(plbm_lattice *h, int steps);
 int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model, int *steps);
@@ -189,8 +193,10 @@ int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model, int *st
  *                       swaps its iold/inew ids once per step, as the reference does).
  *                       It runs in temporally blocked passes
  *                       (plbm_dugks_set_steps_per_pass).  The two slots and the buffer of
- *                       plbm_set_pass_lag_buffer may exchange their device storage (under
- *                       stream capture the two slots only), so addresses from
+ *                       plbm_set_pass_lag_buffer may exchange their device storage (from the
+ *                       first captured call on, see plbm_run, the two slots only, and
+ *                       on grids of fewer than 2048 walks of 64 columns only after an odd
+ *                       number of steps), so addresses from
  *                       plbm_buffer_ptr for them must be fetched again.  Asynchronous. */
 int plbm_dugks_collide(plbm_lattice *h, int src, int dst, double omega_full,
                        double omega_half);
@@ -200,7 +206,7 @@ int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, double dt,
 /* Steps per pass of plbm_dugks_step: 1 = the collide + flux pair every step; 2..3 = all
  * steps but the last in temporally blocked passes of up to this many steps over device
  * memory; 0 (default) = chosen from the grid size, the last pass also storing the
- * half-collided state (plbm_set_pass_lag_buffer; without it, and under stream capture, as
+ * half-collided state (plbm_set_pass_lag_buffer; without it, and after a captured call, as
  * 2..3).  Bit-identical for every value.  The getter returns the depth for equal rates. */
 int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps);
 /* DUGKS as the reference builds it with -DDUGKS (src/periodic_dugks.F90:68,199,267,308):
@@ -281,8 +287,7 @@ int plbm_get_launch(const plbm_lattice *h, int model, int *block, int *xcd_remap
  * grids and by wavefronts walking segments of columns on larger ones; 0 = chosen from the
  * grid size: launches of up to 8 steps (of up to 11 in tiles, as many as make the run
  * cheapest; the get variant reports 8), or single steps on wide, flat grids beyond the
- * tiles' limit, and while the lattice's stream is being captured on grids below about
- * 512^2).  In F64 storage the results are bit-identical for every setting;
+ * tiles' limit, and after a captured call on grids below about 512^2).  In F64 storage the results are bit-identical for every setting;
  * the shifted storages agree to roundoff (their collisions allow FMA contraction, which
  * the compiler places per kernel).  plbm_run keeps the reference's slot contents (latest
  * in *iold, the state one step earlier in *inew); with passes of more than one step it

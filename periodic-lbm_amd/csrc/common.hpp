@@ -313,6 +313,9 @@ struct plbm_lattice {
     void *aux = nullptr;
     bool aux_failed = false;             // its allocation failed once; runs end on a single step
     bool aux_enabled = true;             // plbm_set_pass_lag_buffer
+    // A call that uses a slot was captured (note_capture): runs move the slots' storage only
+    // as they do while being captured, so that the graph's addresses stay the slots'.
+    bool captured = false;
     // per-launch timing of plbm_run (plbm_set_run_timing): events around each launch of
     // the last run and the steps each launch advanced
     bool run_timing = false;
@@ -325,3 +328,13 @@ struct plbm_lattice {
     double *d_partials = nullptr;  // kReduceBlocks * PLBM_NRED
     double *d_red = nullptr;       // PLBM_NRED
 };
+
+namespace plbm {
+// Called by every entry point that uses a slot's storage (53 ns until the first capture).
+inline void note_capture(plbm_lattice *h) {
+    if (h->captured) return;
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &s) != hipSuccess) (void)hipGetLastError();
+    h->captured = s != hipStreamCaptureStatusNone;
+}
+}  // namespace plbm

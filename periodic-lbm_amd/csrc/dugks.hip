@@ -23,7 +23,7 @@
 // per cell and pass, 216 for the last, which also writes the half-collided state into the
 // lattice's third buffer; the three buffers' storage rotates so that slot contents equal the
 // reference's buffers after the same number of perform_dugks_step calls.  Without that buffer,
-// while the stream is captured, and when the caller set the pass depth, the last step is the
+// once a call was captured, and when the caller set the pass depth, the last step is the
 // two-kernel form, the others passes, and the two slots exchange their storage at most.
 // The -DDUGKS build's form (half collision at 0.75 of its rate, which the caller passes,
 // and face collisions in the stream) is plbm_dugks_stream_faces / plbm_dugks_step_faces
@@ -240,6 +240,7 @@ static int dugks_check(plbm_lattice *h, int a, int b) {
                  "need distinct valid buffers");
     PLBM_REQUIRE(h->storage == PLBM_F64, PLBM_ERR_STATE,
                  "the DUGKS operators run on FP64 (PLBM_F64) storage");
+    note_capture(h);
     return PLBM_OK;
 }
 
@@ -419,10 +420,8 @@ extern "C" int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, 
     const int ns = dugks_steps_per_pass(h, two);
     double *latest = static_cast<double *>(h->f[iold]);
     double *other = static_cast<double *>(h->f[inew]);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
-    const bool captured = cap != hipStreamCaptureStatusNone;
-    double *aux = h->dugks_ns == 0 && !captured ? static_cast<double *>(pass_aux(h)) : nullptr;
+    double *aux =
+        h->dugks_ns == 0 && !h->captured ? static_cast<double *>(pass_aux(h)) : nullptr;
     if (aux != nullptr) {
         const std::vector<int> plan =
             dugks_tiles(h, two) ? pass_plan(nsteps, ns) : lag_pass_plan(nsteps, ns);
@@ -439,10 +438,11 @@ extern "C" int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, 
     // All steps but the last in groups, each of one pass, whose buffers change places, and
     // for the steps that it does not reach the collide + flux pair, which stays in place; the
     // last step is the pair, which leaves the half-collided state in the other buffer.  Where
-    // the slots' storage ends depends on the groups only, and a captured run's must not
-    // depend on more than the grid: single steps (in place) below 2048 walks of 64 columns.
+    // the slots' storage ends depends on the groups only, and where a graph holds addresses
+    // (plbm_lattice::captured) it must not depend on more than the grid: single steps (in place)
+    // below 2048 walks of 64 columns.
     const long walks = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
-    const int group = h->dugks_ns > 0 ? h->dugks_ns : !captured ? ns : walks < 2048 ? 1 : 3;
+    const int group = h->dugks_ns > 0 ? h->dugks_ns : !h->captured ? ns : walks < 2048 ? 1 : 3;
     for (int done = 0; done < nsteps - 1;) {
         const int k = std::min(group, nsteps - 1 - done);
         const int in_pass = k > 1 ? std::min(k, ns) : 0;

@@ -280,11 +280,14 @@ static StepArgs make_args(const plbm_lattice *h, const void *src, void *dst,
     return a;
 }
 
-static int check_buf(const plbm_lattice *h, int buf) {
+// Slots of a call: one, or a and b.
+static int check_buf(plbm_lattice *h, int a, int b = 0) {
     PLBM_REQUIRE(h, PLBM_ERR_ARG, "null lattice handle");
-    PLBM_REQUIRE(buf >= 0 && buf < h->nf, PLBM_ERR_ARG,
-                 "buffer id " + std::to_string(buf) + " out of range [0," +
-                     std::to_string(h->nf) + ")");
+    for (int buf : {a, b})
+        PLBM_REQUIRE(buf >= 0 && buf < h->nf, PLBM_ERR_ARG,
+                     "buffer id " + std::to_string(buf) + " out of range [0," +
+                         std::to_string(h->nf) + ")");
+    note_capture(h);
     return PLBM_OK;
 }
 
@@ -757,8 +760,7 @@ int plbm_equilibrium_init(plbm_lattice *h, int buf, const double *rho, const dou
 }
 
 int plbm_step(plbm_lattice *h, int model, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src));
-    PLBM_TRY(check_buf(h, dst));
+    PLBM_TRY(check_buf(h, src, dst));
     PLBM_REQUIRE(src != dst, PLBM_ERR_ARG, "fused step needs distinct src and dst buffers");
     PLBM_TRY(require_params(h));
     return launch_step(h, model, h->f[src], h->f[dst]);
@@ -771,8 +773,7 @@ int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) try {
     PLBM_REQUIRE(nsteps >= 0, PLBM_ERR_ARG, "nsteps must be >= 0");
     PLBM_REQUIRE(model >= PLBM_BGK && model <= PLBM_BGK_SPLIT, PLBM_ERR_ARG,
                  "unknown collision model " + std::to_string(model));
-    PLBM_TRY(check_buf(h, *iold));
-    PLBM_TRY(check_buf(h, *inew));
+    PLBM_TRY(check_buf(h, *iold, *inew));
     PLBM_REQUIRE(*iold != *inew, PLBM_ERR_ARG, "iold == inew");
     PLBM_TRY(require_params(h));
     return run_steps(h, model, nsteps, iold, inew);
@@ -781,8 +782,7 @@ int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) try {
 }
 
 int plbm_stream(plbm_lattice *h, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src));
-    PLBM_TRY(check_buf(h, dst));
+    PLBM_TRY(check_buf(h, src, dst));
     PLBM_REQUIRE(src != dst, PLBM_ERR_ARG, "streaming needs distinct src and dst buffers");
     return dispatch_storage(h->storage, [&](auto S) {
         using T = typename Traits<decltype(S)::value>::T;
@@ -815,8 +815,7 @@ int plbm_collide(plbm_lattice *h, int model, int buf) try {
 }
 
 int plbm_copy(plbm_lattice *h, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src));
-    PLBM_TRY(check_buf(h, dst));
+    PLBM_TRY(check_buf(h, src, dst));
     if (src == dst) return PLBM_OK;
     PLBM_HIP(hipMemcpyAsync(h->f[dst], h->f[src], h->elems * storage_bytes(h->storage),
                             hipMemcpyDeviceToDevice, h->stream));

@@ -275,22 +275,19 @@ static int timing_mark(plbm_lattice *h, int depth) {
 // passes.  On grids of fewer than 512 column walks the passes stand for single steps and
 // round as they do (as_single).  On larger ones FP16 storage, which rounds a state whenever it
 // is stored, keeps the depth of 8.
-// While the stream is being captured, such small grids keep single steps: their slots do not
-// move, so that a caller's graph can be replayed.
+// Once a call was captured (plbm_lattice::captured), such small grids keep single steps, whose
+// slots do not move, and larger ones passes of 8, so that a caller's graph can be replayed, also
+// after further runs.
 int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
     int ns = h->cfg[model].ns, lag_ns = h->cfg[model].lag_ns;
     bool even = false, as_single = false;
     if (ns == 0 && nsteps >= 2) {
         const bool walks = enough_walks(h);
         ns = walks ? kMaxPassSteps : 1;
-        if (tile_grid(h, model) && (!walks || h->storage != PLBM_F16S)) {
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (!walks) PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
-            if (cap == hipStreamCaptureStatusNone) {
-                ns = tile_depth(h->nx, h->ny, tile_kind(h, model), nsteps);
-                even = true;
-                as_single = !walks;
-            }
+        if (tile_grid(h, model) && !h->captured && (!walks || h->storage != PLBM_F16S)) {
+            ns = tile_depth(h->nx, h->ny, tile_kind(h, model), nsteps);
+            even = true;
+            as_single = !walks;
         }
     }
     h->run_depths.clear();
@@ -346,6 +343,7 @@ extern "C" int plbm_pass(plbm_lattice *h, int model, int steps, int src, int dst
                  "need distinct valid src and dst buffers");
     PLBM_REQUIRE(h->params_set, PLBM_ERR_STATE,
                  "collision parameters not set: call plbm_set_params first");
+    note_capture(h);
     if (steps == 1) return launch_step(h, model, h->f[src], h->f[dst]);
     return launch_multi(h, model, steps, h->f[src], h->f[dst]);
 } catch (...) {

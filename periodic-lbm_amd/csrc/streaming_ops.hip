@@ -58,6 +58,7 @@ int check_op_args(plbm_lattice *h, int op, int src, int dst, double dt) {
     PLBM_REQUIRE(std::isfinite(dt), PLBM_ERR_ARG, "non-finite dt");
     PLBM_REQUIRE(op >= PLBM_STREAM_EXACT && op <= PLBM_STREAM_FDM_BARDOW_ISO, PLBM_ERR_ARG,
                  "unknown streaming operator " + std::to_string(op));
+    note_capture(h);
     return PLBM_OK;
 }
 
@@ -82,9 +83,9 @@ extern "C" int plbm_step_op(plbm_lattice *h, int op, int model, int src, int dst
     return plbm::host_exception();
 }
 
-// Whether single steps were the automatic choice before the passes could fill the chip on
-// grids of fewer than 2048 walks of 64 columns: while the stream is captured they still are,
-// as their slots do not move.
+// Grids on which a captured run (plbm_lattice::captured) takes single steps, whose slots do not
+// move; on others it takes passes of 3.  A graph is then replayed from the slots it was captured
+// with, whatever the automatic depth of other runs is.
 static bool fd_few_walks(const plbm_lattice *h) {
     return (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS) < 2048;
 }
@@ -134,12 +135,9 @@ extern "C" int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *
     PLBM_REQUIRE(h->params_set, PLBM_ERR_STATE, "plbm_set_params has not been called");
     if (op == PLBM_STREAM_EXACT) return plbm_run(h, model, nsteps, iold, inew);
     int ns = fd_steps_per_pass(h);
-    const bool even = h->fd_ns == 0 && fd_tile_grid(h);
-    if (h->fd_ns == 0 && ns > 1 && fd_few_walks(h)) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        PLBM_HIP(hipStreamIsCapturing(h->stream, &cap));
-        if (cap != hipStreamCaptureStatusNone) ns = 1;
-    }
+    const bool fixed = h->fd_ns == 0 && h->captured;
+    if (fixed && ns > 1) ns = fd_few_walks(h) ? 1 : 3;
+    const bool even = h->fd_ns == 0 && !fixed && fd_tile_grid(h);
     if (ns <= 1 || nsteps < 2) {
         for (int s = 0; s < nsteps; ++s) {
             PLBM_TRY(launch_fd(h, op, model, h->f[*iold], h->f[*inew], dt));
