@@ -406,7 +406,9 @@ int plbm_adjoint_forward_dev(plbm_adjoint *a, const double *rho0, const double *
                              const double *uy0, double omega, const double *uxt,
                              const double *uyt, double *loss);
 /* Gradients of the last forward's loss: dL/drho0 (may be NULL), dL/dux0, dL/duy0
- * (device, (ny,nx)) and dL/domega (host scalar). */
+ * (device, (ny,nx)) and dL/domega (host scalar).  May be called again after one forward, with
+ * the same results; PLBM_ERR_STATE without a completed forward, and on a further call where
+ * FP32 storage found no memory to keep the adjoint state of f^N. */
 int plbm_adjoint_backward_dev(plbm_adjoint *a, double *grho0, double *gux0, double *guy0,
                               double *gomega);
 

@@ -69,7 +69,8 @@ class Adjoint:
         return loss.value
 
     def backward(self):
-        """Returns (dL/drho0, dL/dux0, dL/duy0, dL/domega) of the last forward()."""
+        """Returns (dL/drho0, dL/dux0, dL/duy0, dL/domega) of the last forward(); may be called
+        again, while the forward's tensors are alive."""
         import torch
         dev = torch.device("cuda")
         g = [torch.empty((self.nx, self.ny), dtype=torch.float64, device=dev) for _ in range(3)]

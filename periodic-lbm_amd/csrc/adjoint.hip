@@ -12,8 +12,8 @@
 //
 // Memory: states are checkpointed every K steps during the forward sweep, which leaves the
 // last K-step segment's states in a segment buffer; the reverse sweep recomputes each earlier
-// segment into it from its checkpoint before it runs the K reverse steps.  Forward cost
-// about 2N - K steps, reverse N steps.
+// segment into it from its checkpoint before it runs the K reverse steps (a further backward
+// call the last one too).  Forward cost about 2N - K steps, reverse N steps.
 //
 // All three run in LDS tiles of several steps: the forward from checkpoint to checkpoint
 // (tile.hip), the recomputation storing every level on its way, the reverse sweep in
@@ -29,6 +29,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "common.hpp"
@@ -371,7 +372,11 @@ struct plbm_adjoint {
     plbm_lattice *lat = nullptr;   // forward buffers (ping-pong) + launch plumbing
     void *checkpoints = nullptr;   // ncheck buffers: f^0, f^K, f^2K, ...
     void *segment = nullptr;       // every buffers: the states of one segment after its first
-    void *mu[2] = {nullptr, nullptr};
+    int held = -1;                 // the segment whose states it holds
+    // The adjoint state: mu[0] of f^N, kept for further backward calls, and the two that a
+    // reverse sweep alternates between (8-byte storages: the lattice's buffers, free by then).
+    // Where FP32 storage has no memory for the third, the sweep overwrites mu[0].
+    void *mu[3] = {nullptr, nullptr, nullptr};
     Sum2 *sums = nullptr;          // omega sensitivity, one per thread of a reverse pass
     size_t nsums = 0;              // the most threads that one has
     size_t buf_bytes = 0, mu_bytes = 0;
@@ -410,11 +415,13 @@ static int adj_depth(const plbm_adjoint *a) {
 // f^{n0+1} .. f^{n0+len} of segment k from its checkpoint.
 static int fill_segment(plbm_adjoint *a, int k, int len) {
     if (len < 1) return PLBM_OK;
+    a->held = -1;
     int j = 0;
     for (int ns : pass_plan(len, adj_depth(a))) {
         PLBM_TRY(launch_tile_levels(a->lat, ns, state(a, k, j), state(a, k, j + 1)));
         j += ns;
     }
+    a->held = k;
     return PLBM_OK;
 }
 // Tiles of a reverse pass of ns steps: shape, columns and rows of the grid of them.
@@ -516,12 +523,21 @@ int plbm_adjoint_create(int nx, int ny, int storage, int nsteps, int checkpoint_
     if (hipMalloc(&a->segment, a->every * a->buf_bytes) != hipSuccess)
         return fail("hipMalloc of the adjoint segment buffer failed");
     if (hipMalloc(&a->mu[0], a->mu_bytes) != hipSuccess ||
-        hipMalloc(&a->mu[1], a->mu_bytes) != hipSuccess ||
         hipMalloc(&a->sums, a->nsums * sizeof(Sum2)) != hipSuccess)
         return fail("hipMalloc of adjoint buffers failed");
+    if (a->mu_bytes == a->buf_bytes) {
+        a->mu[1] = a->lat->f[0];
+        a->mu[2] = a->lat->f[1];
+    } else if (hipMalloc(&a->mu[1], a->mu_bytes) != hipSuccess) {
+        return fail("hipMalloc of adjoint buffers failed");
+    }
     if (hipMalloc(&a->d_partials, kAdjBlocks * sizeof(double)) != hipSuccess ||
         hipMalloc(&a->d_scalar, 2 * sizeof(double)) != hipSuccess)
         return fail("hipMalloc of adjoint scalars failed");
+    if (!a->mu[2] && hipMalloc(&a->mu[2], a->mu_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        a->mu[2] = nullptr;
+    }
     *out = a;
     return PLBM_OK;
 } catch (...) {
@@ -534,7 +550,7 @@ int plbm_adjoint_destroy(plbm_adjoint *a) try {
     if (a->checkpoints) (void)hipFree(a->checkpoints);
     if (a->segment) (void)hipFree(a->segment);
     for (void *p : a->mu)
-        if (p) (void)hipFree(p);
+        if (p && p != a->lat->f[0] && p != a->lat->f[1]) (void)hipFree(p);
     if (a->sums) (void)hipFree(a->sums);
     if (a->d_partials) (void)hipFree(a->d_partials);
     if (a->d_scalar) (void)hipFree(a->d_scalar);
@@ -561,6 +577,7 @@ int plbm_adjoint_forward_dev(plbm_adjoint *a, const double *rho0, const double *
     PLBM_REQUIRE(std::isfinite(omega), PLBM_ERR_ARG, "non-finite omega");
     plbm_lattice *h = a->lat;
     PLBM_TRY(plbm_set_params(h, omega, 0.25));
+    a->forward_done = false;
     a->omega = omega;
     a->rho0 = rho0;
     a->ux0 = ux0;
@@ -616,21 +633,22 @@ int plbm_adjoint_backward_dev(plbm_adjoint *a, double *grho0, double *gux0, doub
                        a->stream, reinterpret_cast<double *>(a->sums), 2 * a->nsums);
     PLBM_HIP(hipGetLastError());
     const int depth = adj_depth(a);
-    int cur = 0;  // mu[cur] holds the adjoint state
+    void *in = a->mu[0], *to = a->mu[1], *next = a->mu[2] ? a->mu[2] : a->mu[0];
+    if (!a->mu[2]) a->forward_done = false;
     for (int k = a->ncheck - 1; k >= 0; --k) {
         const int n0 = k * a->every, n1 = std::min(a->nsteps, n0 + a->every);
-        if (k + 1 < a->ncheck) PLBM_TRY(fill_segment(a, k, n1 - n0 - 1));
+        if (a->held != k) PLBM_TRY(fill_segment(a, k, n1 - n0 - 1));
         int top = n1 - 1 - n0;
         for (int ns : pass_plan(n1 - n0, depth)) {
-            PLBM_TRY(launch_adj(a, ns, state(a, k, top), state(a, k, top - ns + 1), a->mu[cur],
-                                a->mu[cur ^ 1]));
-            cur ^= 1;
+            PLBM_TRY(launch_adj(a, ns, state(a, k, top), state(a, k, top - ns + 1), in, to));
+            in = to;
+            std::swap(to, next);
             top -= ns;
         }
     }
     // lambda^0 -> gradients of the initial fields
     hipLaunchKernelGGL(k_adj_initial, dim3((a->ny + 255) / 256, a->nx), dim3(256), 0, a->stream,
-                       static_cast<const double *>(a->mu[cur]), a->nx, a->ny, h->ldd, a->rho0,
+                       static_cast<const double *>(in), a->nx, a->ny, h->ldd, a->rho0,
                        a->ux0, a->uy0, grho0, gux0, guy0);
     PLBM_HIP(hipGetLastError());
     Sum2 *part = reinterpret_cast<Sum2 *>(a->d_partials);
