@@ -326,8 +326,10 @@ int plbm_run_launch_times(plbm_lattice *h, int max_launches, int *depths, float 
                           int *nlaunches);
 /* Autotuner: time every launch shape of the fused step for `model` (reps launches from
  * buffer buf into a scratch buffer; the lattice's buffers are not modified), then passes
- * of 2..8 steps against it per lattice update; keep the fastest for this lattice and
- * cache it per (device, storage, model, grid) for the process.  With passes, it also
+ * of 2..8 steps against it per lattice update (on grids whose runs choose the depth of their
+ * tiles, see plbm_set_steps_per_launch, that choice, which then stays automatic); keep the
+ * fastest for this lattice and cache it for the process per device, storage, model, grid,
+ * column segments, third buffer on or off and captured or not.  With passes, it also
  * times the pass that ends a run (the one that also stores the lagged state, into the
  * lattice's third buffer, allocated here if needed) at every depth from the chosen one
  * up, and keeps for it the depth that makes runs cheapest; plbm_set_steps_per_launch

@@ -272,6 +272,7 @@ int launch_multi(plbm_lattice *h, int model, int ns, const void *src, void *dst,
 // FP32 arithmetic; other passes round FP16 once and compute FP32 BGK in FP64).
 bool tile_grid(const plbm_lattice *h, int model);
 bool tile_cells(int storage, int model, long long cells);
+bool tile_plans(const plbm_lattice *h, int model, bool *as_single);
 int launch_tile(plbm_lattice *h, int model, int ns, const void *src, void *dst, void *lag,
                 bool as_single);
 // One pass of ns >= 1 BGK steps that stores every level (F64, F64S, F32S storage), the roundings

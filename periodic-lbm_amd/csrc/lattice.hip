@@ -23,6 +23,7 @@
 #include "d2q9.hpp"
 #include "reduce.hpp"
 #include "stepper.hpp"
+#include "tile.hpp"
 
 namespace plbm {
 
@@ -413,14 +414,16 @@ static bool valid_cfg(LaunchCfg c) {
 // (device, storage, model, grid) by timing every candidate with HIP events on the
 // lattice's stream: `reps` launches from buffer src into a scratch buffer (so the
 // lattice's own state is untouched), best of three trials each.  Results are cached per
-// process, keyed by device name, storage, model and grid size.
+// process, keyed by device name, storage, model, grid size and what else decides which kernels
+// a run takes: the column segments, the third buffer and whether a call was captured.
 
 struct TuneKey {
     std::string dev;
-    int storage, model, nx, ny;
+    int storage, model, nx, ny, segs;
+    bool aux, captured;
     bool operator<(const TuneKey &o) const {
-        return std::tie(dev, storage, model, nx, ny) <
-               std::tie(o.dev, o.storage, o.model, o.nx, o.ny);
+        return std::tie(dev, storage, model, nx, ny, segs, aux, captured) <
+               std::tie(o.dev, o.storage, o.model, o.nx, o.ny, o.segs, o.aux, o.captured);
     }
 };
 static std::map<TuneKey, std::pair<LaunchCfg, double>> g_tune_cache;
@@ -434,7 +437,8 @@ static std::string device_name(int dev) {
 
 int autotune_step(plbm_lattice *h, int model, int src, int reps, LaunchCfg *best_out,
                   double *best_ms) {
-    TuneKey key{device_name(h->device), h->storage, model, h->nx, h->ny};
+    TuneKey key{device_name(h->device), h->storage, model,        h->nx, h->ny,
+                h->pass_segs,           h->aux_enabled, h->captured};
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune_cache.find(key);
@@ -496,9 +500,27 @@ int autotune_step(plbm_lattice *h, int model, int src, int reps, LaunchCfg *best
         }
     }
     // steps per pass of plbm_run: the single-step kernel at the shape just chosen against
-    // passes of 2..8 steps, compared per lattice update
+    // passes of 2..8 steps, compared per lattice update; or, where runs choose the depth of
+    // their tiles (up to 11, for each run's length), against that choice, which stays with them
     best.ns = 1;
-    for (int ns = 2; ns <= max_steps_per_pass(h->storage); ++ns) {
+    bool as_single;
+    const bool plans = tile_plans(h, model, &as_single);
+    if (plans) {
+        int shape = 0, ns = 2;
+        pick_tile(h->nx, h->ny, tile_kind(h, model), 2, kMaxTileSteps, &shape, &ns);
+        double t;
+        PLBM_TRY(time_launch(
+            [&] {
+                return launch_tile(h, model, ns, h->f[src], scratch, nullptr, as_single);
+            },
+            &t));
+        if (t / ns < tbest) {
+            tbest = t / ns;
+            best.ns = 0;
+            (void)pass_aux(h);  // runs will need it
+        }
+    }
+    for (int ns = plans ? max_steps_per_pass(h->storage) + 1 : 2; ns <= max_steps_per_pass(h->storage); ++ns) {
         double t;
         PLBM_TRY(time_launch([&] { return launch_multi(h, model, ns, h->f[src], scratch); }, &t));
         if (t / ns < tbest) {

@@ -103,6 +103,14 @@ static bool enough_walks(const plbm_lattice *h) {
     return (long)((h->ny + vr - 1) / vr) * walk_segments(h->nx) >= 512;
 }
 
+// Whether runs at the automatic depth take tiles of the depth that is cheapest for their length:
+// not on the larger of those grids in FP16 storage (run_steps), nor once a call was captured.
+bool tile_plans(const plbm_lattice *h, int model, bool *as_single) {
+    const bool walks = enough_walks(h);
+    *as_single = !walks;
+    return tile_grid(h, model) && !h->captured && (!walks || h->storage != PLBM_F16S);
+}
+
 // Most steps of a launch of plbm_run when the caller has not chosen, as reported: 8 where it
 // runs in tiles (which go to 11, see run_steps), or where the column walk has at least 512
 // wavefronts; else single steps (wide and flat grids beyond the tiles' limit).
@@ -282,13 +290,9 @@ int run_steps(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) {
     int ns = h->cfg[model].ns, lag_ns = h->cfg[model].lag_ns;
     bool even = false, as_single = false;
     if (ns == 0 && nsteps >= 2) {
-        const bool walks = enough_walks(h);
-        ns = walks ? kMaxPassSteps : 1;
-        if (tile_grid(h, model) && !h->captured && (!walks || h->storage != PLBM_F16S)) {
-            ns = tile_depth(h->nx, h->ny, tile_kind(h, model), nsteps);
-            even = true;
-            as_single = !walks;
-        }
+        even = tile_plans(h, model, &as_single);
+        ns = even ? tile_depth(h->nx, h->ny, tile_kind(h, model), nsteps)
+                  : enough_walks(h) ? kMaxPassSteps : 1;
     }
     h->run_depths.clear();
     PLBM_TRY(timing_mark(h, 0));
