@@ -175,7 +175,7 @@ int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *iold, int *
  * 0 = chosen from the grid size (FP64: passes of up to 6 steps, in LDS tiles on small grids
  * and by column walks on larger ones; from the first captured call on, see plbm_run, single
  * steps on grids of fewer than 2048 walks of 64 columns, else 3).  The get variant reports the
- * effective value for (op, model). */
+ * effective value for (op, model) as far as it can be set: 3 where the choice is deeper. */
 int plbm_set_op_steps_per_pass(plbm_lattice *h, int steps);
 int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int model, int *steps);
 
@@ -207,7 +207,8 @@ int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, double dt,
  * steps but the last in temporally blocked passes of up to this many steps over device
  * memory; 0 (default) = chosen from the grid size, the last pass also storing the
  * half-collided state (plbm_set_pass_lag_buffer; without it, and after a captured call, as
- * 2..3).  Bit-identical for every value.  The getter returns the depth for equal rates. */
+ * 2..3).  Bit-identical for every value.  The getter returns the depth for equal rates as
+ * far as it can be set: 3 where the choice is deeper. */
 int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps);
 /* DUGKS as the reference builds it with -DDUGKS (src/periodic_dugks.F90:68,199,267,308):
  * the stream relaxes the interpolated face values of every face towards the face's own

@@ -403,7 +403,7 @@ extern "C" int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps) try {
 
 extern "C" int plbm_dugks_get_steps_per_pass(const plbm_lattice *h, int *steps) try {
     PLBM_REQUIRE(h && steps, PLBM_ERR_ARG, "null argument");
-    *steps = dugks_steps_per_pass(h, false);
+    *steps = std::min(dugks_steps_per_pass(h, false), 3);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();

@@ -14,6 +14,7 @@
 // scaled storage directly.  FP64 expression trees follow the reference with FMA
 // contraction off, which makes them bit-identical to it.  The reference loops x over ny
 // and y over nx (square grids); here x runs over nx and y over ny.
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -119,7 +120,7 @@ extern "C" int plbm_get_op_steps_per_pass(const plbm_lattice *h, int op, int mod
     PLBM_REQUIRE(h && steps, PLBM_ERR_ARG, "null argument");
     (void)op;
     (void)model;
-    *steps = fd_steps_per_pass(h);
+    *steps = std::min(fd_steps_per_pass(h), 3);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();
