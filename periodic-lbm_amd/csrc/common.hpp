@@ -331,9 +331,10 @@ struct plbm_lattice {
 };
 
 namespace plbm {
-// Called by every entry point that uses a slot's storage (53 ns until the first capture).
+// Called by every entry point that uses a slot's storage.  A lattice's own stream is nobody else's
+// to capture; asking on every call cost 0.25 of 4.7 us per step.
 inline void note_capture(plbm_lattice *h) {
-    if (h->captured) return;
+    if (h->captured || h->stream == h->own) return;
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(h->stream, &s) != hipSuccess) (void)hipGetLastError();
     h->captured = s != hipStreamCaptureStatusNone;
