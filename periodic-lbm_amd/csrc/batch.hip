@@ -314,7 +314,7 @@ struct plbm_batch {
     // cached graphs: key = (nsteps, parity at start)
     std::map<std::pair<int, int>, hipGraphExec_t> graphs;
     double *d_red = nullptr;
-    HostStage stage;  // read-back of small fields
+    HostStageUser stage_user;
     double *d_tmp = nullptr;
     size_t tmp_bytes = 0;
 };
@@ -698,7 +698,6 @@ int plbm_batch_destroy(plbm_batch *b) try {
     if (b->d_cases) (void)hipFree(b->d_cases);
     if (b->d_red) (void)hipFree(b->d_red);
     if (b->d_tmp) (void)hipFree(b->d_tmp);
-    b->stage.release();
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->join) (void)hipEventDestroy(b->join);
     if (b->side) (void)hipStreamDestroy(b->side);
@@ -835,8 +834,8 @@ int plbm_batch_macros(plbm_batch *b, int c, double *rho, double *ux, double *uy)
             return PLBM_OK;
         });
     };
-    if (b->stage.ready(3 * n * sizeof(double)))
-        return fields_through_stage(b->stage, b->stream, k.nx, k.ny, launch, rho, ux, uy);
+    if (HostStage stage(3 * n * sizeof(double)); stage)
+        return fields_through_stage(stage, b->stream, k.nx, k.ny, launch, rho, ux, uy);
     PLBM_TRY(ensure_btmp(b, 3 * n * sizeof(double)));
     PLBM_TRY(launch(0, (size_t)k.nx, b->d_tmp, b->d_tmp + n, b->d_tmp + 2 * n));
     PLBM_HIP(hipMemcpyAsync(rho, b->d_tmp, n * 8, hipMemcpyDeviceToHost, b->stream));

@@ -206,37 +206,35 @@ inline int plane_from_host(double *dev, const double *host, size_t ld, size_t ny
 
 // Pinned memory through which small fields reach the caller's pageable arrays: a kernel stores
 // them there over the bus, in two halves so that one half's copy on the host overlaps the
-// other's transfer.  Kept by its lattice or batch.  Reading three fields back took, by three
-// copies into pageable memory, at 64^2 / 128^2 / 200^2 / 256^2 / 320^2, 81 / 59 / 83 / 108 / 146
-// us; this 30 / 40 / 60 / 80 / 110.  Larger fields keep the copies, which fault fresh pages in
-// in bulk (512^2 450 us, against 3.6 ms of page faults in a copy on the host).  1 MiB takes 45
-// us to allocate, the most, 2.5 MiB, 280: hence two sizes.
-struct HostStage {
-    void *mem = nullptr;
-    size_t bytes = 0;
+// other's transfer.  Reading three fields back takes, by three copies into pageable memory, at
+// 64^2 / 128^2 / 200^2 / 256^2 / 320^2, 47 / 61 / 89 / 120 / 162 us; this 30 / 41 / 61 / 81 / 111.
+// Larger fields keep the copies, which fault fresh pages in in bulk (512^2 450 us, against 3.6 ms
+// of page faults in a copy on the host).
+//
+// A block of 1 MiB takes 35 to 130 us to allocate, one of 2.5 MiB 280 to 500.  The process
+// therefore has one of each, allocated when as many reads were made by copies as it costs, and
+// freed with the last lattice or batch; a HostStage holds one for the length of a call that waits
+// for its stream, and a call that finds it taken by another thread copies.  A block per lattice
+// instead made the first reads slower: 40 lattices of 64^2 read twice, ms, by copies 7.0, with a
+// block each 8.0, so 2.6; of 320^2 67, 51, 10.
+class HostStage {
+public:
+    explicit HostStage(size_t need);
+    ~HostStage();
+    HostStage(const HostStage &) = delete;
+    explicit operator bool() const { return mem != nullptr; }
+
+    double *mem = nullptr;
     hipEvent_t half = nullptr;
-    bool failed = false;
-    bool ready(size_t need) {
-        const size_t small = (size_t)1 << 20, most = (size_t)5 << 19;
-        if (need > most || failed) return false;
-        if (bytes >= need) return true;
-        release();
-        bytes = need > small ? most : small;
-        if (hipHostMalloc(&mem, bytes, hipHostMallocDefault) != hipSuccess ||
-            hipEventCreateWithFlags(&half, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            release();
-            failed = true;
-        }
-        return !failed;
-    }
-    void release() {
-        if (half) (void)hipEventDestroy(half);
-        if (mem) (void)hipHostFree(mem);
-        mem = nullptr;
-        bytes = 0;
-        half = nullptr;
-    }
+
+private:
+    int size = 0;
+};
+// Held by every lattice and batch: the blocks are freed with the last.
+struct HostStageUser {
+    HostStageUser();
+    ~HostStageUser();
+    HostStageUser(const HostStageUser &) = delete;
 };
 
 // Three fields of nx columns of ny into host arrays; launch(x0, columns, rho, ux, uy) issues
@@ -244,7 +242,12 @@ struct HostStage {
 template <class F>
 inline int fields_through_stage(HostStage &st, hipStream_t s, size_t nx, size_t ny, F &&launch,
                                 double *rho, double *ux, double *uy) {
-    double *m = static_cast<double *>(st.mem);
+    double *m = st.mem;
+    // after an error as well, nothing writes into the block once another call may have it
+    bool idle = false;
+    auto wait = on_scope_exit([&] {
+        if (!idle) (void)hipStreamSynchronize(s);
+    });
     const size_t x1 = nx / 2, n = nx * ny, n1 = x1 * ny;
     if (x1 > 0) PLBM_TRY(launch((size_t)0, x1, m, m + n, m + 2 * n));
     PLBM_HIP(hipEventRecord(st.half, s));
@@ -253,6 +256,7 @@ inline int fields_through_stage(HostStage &st, hipStream_t s, size_t nx, size_t 
     PLBM_HIP(hipEventSynchronize(st.half));
     for (int c = 0; c < 3; ++c) std::copy(m + c * n, m + c * n + n1, out[c]);
     PLBM_HIP(hipStreamSynchronize(s));
+    idle = true;
     for (int c = 0; c < 3; ++c) std::copy(m + c * n + n1, m + (c + 1) * n, out[c] + n1);
     return PLBM_OK;
 }
@@ -322,8 +326,8 @@ struct plbm_lattice {
     bool run_timing = false;
     std::vector<hipEvent_t> run_events;
     std::vector<int> run_depths;
+    plbm::HostStageUser stage_user;
     // scratch (allocated on first use)
-    plbm::HostStage stage;         // read-back of small fields
     double *d_tmp = nullptr;       // staging for host transfers
     size_t tmp_bytes = 0;
     double *d_partials = nullptr;  // kReduceBlocks * PLBM_NRED

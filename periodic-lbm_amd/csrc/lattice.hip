@@ -408,6 +408,71 @@ static bool valid_cfg(LaunchCfg c) {
     return c.block >= 64 && c.block <= 1024 && c.block % 64 == 0 && (c.remap == 0 || c.remap == 1);
 }
 
+// ------------------------------------------------------------------- pinned read-back blocks
+
+namespace {
+struct StageBlock {
+    size_t bytes;
+    int paid;  // reads by copies after which allocating it would have paid
+    void *mem = nullptr;
+    int reads = 0;
+    bool busy = false, failed = false;
+};
+std::mutex g_stage_mu;
+int g_stage_users = 0;
+StageBlock g_stage[2] = {{(size_t)1 << 20, 4}, {(size_t)5 << 19, 12}};
+}  // namespace
+
+HostStage::HostStage(size_t need) {
+    size = need > g_stage[0].bytes;
+    StageBlock &b = g_stage[size];
+    if (need > b.bytes) return;
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    if (b.busy || b.failed) return;
+    if (!b.mem) {
+        if (b.reads < b.paid) {
+            ++b.reads;
+            return;
+        }
+        if (hipHostMalloc(&b.mem, b.bytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            b.mem = nullptr;
+            b.failed = true;
+            return;
+        }
+        b.paid = 1;  // allocated again after it was freed it takes 10 to 35 us
+    }
+    if (hipEventCreateWithFlags(&half, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    b.busy = true;
+    mem = static_cast<double *>(b.mem);
+}
+
+HostStage::~HostStage() {
+    if (!mem) return;
+    (void)hipEventDestroy(half);
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    g_stage[size].busy = false;
+}
+
+HostStageUser::HostStageUser() {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    ++g_stage_users;
+}
+
+HostStageUser::~HostStageUser() {
+    std::lock_guard<std::mutex> lk(g_stage_mu);
+    if (--g_stage_users > 0) return;
+    for (StageBlock &b : g_stage) {
+        if (b.mem) (void)hipHostFree(b.mem);
+        b.mem = nullptr;
+        b.reads = 0;
+        b.failed = false;
+    }
+}
+
 // ---------------------------------------------------------------------------- autotuner
 //
 // Picks the fused kernel's launch shape (workgroup size x XCD renumbering) for one
@@ -631,7 +696,6 @@ int plbm_destroy(plbm_lattice *h) try {
     for (int b = 0; b < kMaxBuffers; ++b)
         if (h->f[b]) (void)hipFree(h->f[b]);
     if (h->aux) (void)hipFree(h->aux);
-    h->stage.release();
     for (hipEvent_t e : h->run_events) (void)hipEventDestroy(e);
     if (h->d_tmp) (void)hipFree(h->d_tmp);
     if (h->d_partials) (void)hipFree(h->d_partials);
@@ -871,9 +935,9 @@ int plbm_macros(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) t
     PLBM_TRY(check_buf(h, buf));
     PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
     const size_t n = (size_t)h->nx * h->ny;
-    if (h->stage.ready(3 * n * sizeof(double)))
+    if (HostStage stage(3 * n * sizeof(double)); stage)
         return fields_through_stage(
-            h->stage, h->stream, h->nx, h->ny,
+            stage, h->stream, h->nx, h->ny,
             [&](size_t x0, size_t cols, double *r, double *u, double *v) {
                 return launch_macros(h, buf, x0, cols, r, u, v);
             },
