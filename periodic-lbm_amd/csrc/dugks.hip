@@ -356,8 +356,21 @@ namespace plbm {
 constexpr int kDugksWalkOne = 3, kDugksWalkTwo = 2;
 constexpr long long kDugksTileCellsTwo = 500000;
 
+// Long grids of few columns: us per step in runs of 1 / 4 / 40 steps, pair and tiles: unequal rates
+// 1 x 25000 20.5 / 12.3 / 9.4, 27 / 14.6 / 12.0, 4 x 60000 35 / 27 / 25, 50 / 33 / 30; but 6 x
+// 25000 28 / 23 / 20, 31 / 16 / 13; equal ones as the operators (2 x 60000 28 / 21 / 18, 30 / 18 /
+// 15).
+static bool dugks_slender(const plbm_lattice *h, bool two) {
+    return two ? h->nx <= 4 && h->ny > 16384 : fd_slender(h);
+}
 static bool dugks_tiles(const plbm_lattice *h, bool two) {
-    return two ? (long long)h->nx * h->ny <= kDugksTileCellsTwo : fd_tile_grid(h);
+    return two ? (long long)h->nx * h->ny <= kDugksTileCellsTwo && !dugks_slender(h, two)
+               : fd_tile_grid(h);
+}
+// Steps of a group (see plbm_dugks_step) on grids that keep the pair, and after a captured call.
+static int dugks_fixed_group(const plbm_lattice *h) {
+    const long walks = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
+    return walks < 2048 ? 1 : 3;
 }
 
 // Steps per pass: the caller's choice as far as the walks go, or the deepest walk, or tiles of
@@ -403,7 +416,8 @@ extern "C" int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps) try {
 
 extern "C" int plbm_dugks_get_steps_per_pass(const plbm_lattice *h, int *steps) try {
     PLBM_REQUIRE(h && steps, PLBM_ERR_ARG, "null argument");
-    *steps = std::min(dugks_steps_per_pass(h, false), 3);
+    const bool fixed = h->dugks_ns == 0 && (h->captured || dugks_slender(h, false));
+    *steps = fixed ? dugks_fixed_group(h) : std::min(dugks_steps_per_pass(h, false), 3);
     return PLBM_OK;
 } catch (...) {
     return plbm::host_exception();
@@ -420,8 +434,8 @@ extern "C" int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, 
     const int ns = dugks_steps_per_pass(h, two);
     double *latest = static_cast<double *>(h->f[iold]);
     double *other = static_cast<double *>(h->f[inew]);
-    double *aux =
-        h->dugks_ns == 0 && !h->captured ? static_cast<double *>(pass_aux(h)) : nullptr;
+    const bool fixed = h->captured || dugks_slender(h, two);
+    double *aux = h->dugks_ns == 0 && !fixed ? static_cast<double *>(pass_aux(h)) : nullptr;
     if (aux != nullptr) {
         const std::vector<int> plan =
             dugks_tiles(h, two) ? pass_plan(nsteps, ns) : lag_pass_plan(nsteps, ns);
@@ -441,8 +455,7 @@ extern "C" int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, 
     // the slots' storage ends depends on the groups only, and where a graph holds addresses
     // (plbm_lattice::captured) it must not depend on more than the grid: single steps (in place)
     // below 2048 walks of 64 columns.
-    const long walks = (long)((h->ny + 55) / 56) * ((h->nx + kMultiXS - 1) / kMultiXS);
-    const int group = h->dugks_ns > 0 ? h->dugks_ns : !h->captured ? ns : walks < 2048 ? 1 : 3;
+    const int group = h->dugks_ns > 0 ? h->dugks_ns : fixed ? dugks_fixed_group(h) : ns;
     for (int done = 0; done < nsteps - 1;) {
         const int k = std::min(group, nsteps - 1 - done);
         const int in_pass = k > 1 ? std::min(k, ns) : 0;

@@ -623,8 +623,15 @@ int launch_fd_walk(plbm_lattice *h, const StepArgs &a, const FdScalars &sc) {
     return PLBM_OK;
 }
 
+// Long grids of few columns, whose tiles are mostly halo, keep single steps: us per step, FVM + BGK,
+// runs of 4 / 40 steps, single steps and tiles: 1 x 25000 8.0 / 5.4, 9.6 / 6.9, 2 x 60000 11.8 /
+// 9.3, 17.5 / 14.6, 4 x 60000 18.7 / 16.0, 19.4 / 16.4; but 3 x 25000 11.3 / 8.7, 9.9 / 7.1, 6 x
+// 60000 26 / 23, 19.7 / 16.9.
+inline bool fd_slender(const plbm_lattice *h) {
+    return h->nx <= 4 && h->ny > 8192 * (h->nx + 1);
+}
 inline bool fd_tile_grid(const plbm_lattice *h) {
-    return (long long)h->nx * h->ny <= kFdTileCells;
+    return (long long)h->nx * h->ny <= kFdTileCells && !fd_slender(h);
 }
 
 // One pass of ns steps (2 .. kFdTileSteps in tiles, 2 .. kFdWalkSteps in walks) of operator

@@ -98,6 +98,7 @@ static bool fd_few_walks(const plbm_lattice *h) {
 static int fd_steps_per_pass(const plbm_lattice *h) {
     if (h->fd_ns > 0) return h->fd_ns;
     if (h->storage != PLBM_F64) return 1;
+    if (fd_slender(h) && fd_few_walks(h)) return 1;
     if (!fd_tile_grid(h)) return kFdWalkSteps;
     int shape, ns = 2;
     pick_fd_tile(h->nx, h->ny, 2, kFdTileSteps, false, &shape, &ns);

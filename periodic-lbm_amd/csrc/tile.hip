@@ -98,9 +98,15 @@ bool tile_cells(int storage, int model, long long cells) {
     return pick(1400000, 850000, 2200000);
 }
 
-// A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.
+// Long grids of few columns are mostly halo as tiles, and give the column walk a wavefront per
+// band: us per step in runs of 4 / 40 steps, walks and tiles: 1 x 60000 BGK FP64 6.8 / 7.1, 9.3 /
+// 6.4, TRT FP32 4.9 / 2.9, 6.2 / 3.4, 2 x 200000 FP64 12.1 / 18.3, 25 / 22, 8 x 60000 BGK FP32
+// 7.9 / 5.2, 9.0 / 6.1; but 1 x 25000 BGK FP64 5.9 / 3.8, 5.5 / 3.3, 6 x 60000 10.0 / 10.1, 11.2 /
+// 8.3.  A caller who chose the column walk's segments (plbm_set_pass_segments) keeps it.
 bool tile_grid(const plbm_lattice *h, int model) {
-    return h->pass_segs == 0 && tile_cells(h->storage, model, (long long)h->nx * h->ny);
+    const bool slender = h->ny > 32768 && h->nx <= (h->storage == PLBM_F32S ? 8 : 4);
+    return h->pass_segs == 0 && !slender &&
+           tile_cells(h->storage, model, (long long)h->nx * h->ny);
 }
 
 static StepArgs tile_args(const plbm_lattice *h, const void *src, void *dst, void *lag) {
