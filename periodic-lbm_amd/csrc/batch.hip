@@ -345,10 +345,19 @@ static bool batch_tile_cells(int storage, int model, long long cells) {
 // instead: TRT FP64 5.9 -> 6.9 us per step at 0.7 M cells, RR FP32 4.9 -> 5.2.
 static int pass_shape(const plbm_batch *b, const BatchCfg &cfg) {
     if (cfg.ns < 2 || cfg.walk || tile_wide(b->storage, b->model)) return -1;
-    long long cells = 0;
-    for (const BatchCase &k : b->cases)
-        if ((long long)k.nx * k.ny > cfg.resident_cells) cells += (long long)k.nx * k.ny;
-    if (!batch_tile_cells(b->storage, b->model, cells)) return -1;
+    // Cases of few columns are mostly halo as tiles: batches of mostly such cases walk, too.  us
+    // per 48 steps in passes of 2 / 4 / 6 / 8, walk and tiles: 40 of 4 x 2000 TRT FP32 211 / - /
+    // 160 / 165, 197 / - / 184 / 216, BGK FP64 379 / - / 306 / 420, 421 / - / 388 / 490; tiles over
+    // walk 1.2-1.6 for 20 of 2 x 8000, 1.1-1.4 for 4 x 8000, 0.7-1.2 for 8 x 8000; 0.8-1.4 for 100
+    // of 1 x 500, 0.7-1.1 of 4 x 500, 0.8-1.1 for 60 of 4 x 1000.
+    long long cells = 0, slender = 0;
+    for (const BatchCase &k : b->cases) {
+        const long long n = (long long)k.nx * k.ny;
+        if (n <= cfg.resident_cells) continue;
+        cells += n;
+        if (k.nx < 8 && k.ny >= 400 * k.nx) slender += n;
+    }
+    if (2 * slender > cells || !batch_tile_cells(b->storage, b->model, cells)) return -1;
     const TileKind kind{(int)storage_bytes(b->storage), b->model};
     int best = -1;
     double cost = 1e300;
