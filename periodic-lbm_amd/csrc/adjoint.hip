@@ -177,11 +177,16 @@ struct Sum2 {
     // an infinite sum's error term is NaN
     __device__ __forceinline__ double value() const { return isfinite(hi) ? hi + lo : hi; }
 };
+// Sum over the calling wavefront.
+__device__ __forceinline__ Sum2 wave_sum(Sum2 v) {
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) v.add({__shfl_xor(v.hi, st), __shfl_xor(v.lo, st)});
+    return v;
+}
 // Sum over the calling workgroup of NT threads, valid in thread 0; sh holds NT / 64 values.
 template <int NT>
 __device__ __forceinline__ Sum2 block_sum(Sum2 v, Sum2 *sh) {
-#pragma unroll
-    for (int st = 32; st > 0; st >>= 1) v.add({__shfl_xor(v.hi, st), __shfl_xor(v.lo, st)});
+    v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0)
@@ -195,7 +200,9 @@ __device__ __forceinline__ Sum2 block_sum(Sum2 v, Sum2 *sh) {
 // cells; an even level gathers from (x + c_q, q) and leaves mu_p where the opposite direction
 // was read, an odd one reads (x, opposite(p)) and writes (x, p).  Level l takes g from state
 // top - (l - 1) stride, the last from `last`.  The omega sensitivity of the tile's own cells is
-// added to the thread's partial sum (a sum over the workgroup per pass took 3-4 us).
+// added to the wavefront's partial sum (a sum over the workgroup per pass took 3-4 us; partial
+// sums of the threads took 142 MB beside states of 29 MB at 1 x 400000, and their traffic: 512^2,
+// 500 steps 6.55 -> 6.50 ms).
 //
 // Bound by its reads of the states, 1.5 times the tile's own with the halo: at 512^2 4.5 TB/s
 // from beyond the L2s, with 42% of the issue slots used.  The whole backward call, 500 steps at
@@ -260,7 +267,9 @@ __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4
                                      const char, char>;
         return reinterpret_cast<decltype(p)>(reinterpret_cast<C *>(p + q * L) + wide * o);
     };
-    Sum2 *mine = a.partials + (size_t)blockIdx.x * NT + threadIdx.x, sum = *mine;
+    Sum2 *mine = a.partials + (size_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+    const bool first_lane = (threadIdx.x & 63) == 0;
+    Sum2 sum = first_lane ? *mine : Sum2{0.0, 0.0};
     auto level = [&](int k, auto first, auto odd) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first)::value, ODD = decltype(odd)::value;
         const T *__restrict__ s = k == ns ? a.last : a.top - (size_t)(k - 1) * a.stride;
@@ -304,7 +313,8 @@ __global__ void __launch_bounds__(SHAPE::T) __attribute__((amdgpu_waves_per_eu(4
         if (k & 1) level(k, no, yes);
         else level(k, no, no);
     }
-    *mine = sum;
+    sum = wave_sum(sum);
+    if (first_lane) *mine = sum;
 }
 
 // One partial sum per workgroup, or of one workgroup the total.
@@ -377,8 +387,8 @@ struct plbm_adjoint {
     // reverse sweep alternates between (8-byte storages: the lattice's buffers, free by then).
     // Where FP32 storage has no memory for the third, the sweep overwrites mu[0].
     void *mu[3] = {nullptr, nullptr, nullptr};
-    Sum2 *sums = nullptr;          // omega sensitivity, one per thread of a reverse pass
-    size_t nsums = 0;              // the most threads that one has
+    Sum2 *sums = nullptr;          // omega sensitivity, one per wavefront of a reverse pass
+    size_t nsums = 0;              // the most wavefronts that one has
     size_t buf_bytes = 0, mu_bytes = 0;
     double omega = 0;
     bool forward_done = false;
@@ -432,11 +442,11 @@ static void adj_tiles(const plbm_adjoint *a, int ns, int *shape, int *nbx, int *
     *nbx = (a->nx + wx - 1) / wx;
     *nby = (a->ny + wy - 1) / wy;
 }
-static size_t adj_threads(const plbm_adjoint *a, int ns) {
+static size_t adj_waves(const plbm_adjoint *a, int ns) {
     int shape = 0, nbx, nby;
     adj_tiles(a, ns, &shape, &nbx, &nby);
     const int t = dispatch_tile_shape(shape, [](auto s) { return decltype(s)::T; });
-    return (size_t)nbx * nby * t;
+    return (size_t)nbx * nby * (t / 64);
 }
 
 // One pass of ns reverse steps, states f^{top} (at `top`) down to the one at `last`.
@@ -511,7 +521,7 @@ int plbm_adjoint_create(int nx, int ny, int storage, int nsteps, int checkpoint_
     a->buf_bytes = a->lat->elems * storage_bytes(storage);
     a->mu_bytes = a->lat->elems * sizeof(double);  // FP64 adjoint state for every storage
     for (int ns = 1; ns <= adj_depth(a); ++ns)
-        a->nsums = std::max(a->nsums, adj_threads(a, ns));
+        a->nsums = std::max(a->nsums, adj_waves(a, ns));
     auto fail = [&](const char *m) {
         (void)hipGetLastError();
         set_error(m);
