@@ -335,8 +335,8 @@ struct plbm_lattice {
 };
 
 namespace plbm {
-// Called by every entry point that uses a slot's storage.  A lattice's own stream is nobody else's
-// to capture; asking on every call cost 0.25 of 4.7 us per step.
+// Called by every entry point that a graph can hold a slot's address of.  A lattice's own stream is
+// nobody else's to capture; asking there as well cost 0.25 of 4.7 us per step.
 inline void note_capture(plbm_lattice *h) {
     if (h->captured || h->stream == h->own) return;
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;

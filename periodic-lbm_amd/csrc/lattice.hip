@@ -281,13 +281,18 @@ static StepArgs make_args(const plbm_lattice *h, const void *src, void *dst,
     return a;
 }
 
-// Slots of a call: one, or a and b.
-static int check_buf(plbm_lattice *h, int a, int b = 0) {
+static int check_buf(const plbm_lattice *h, int buf) {
     PLBM_REQUIRE(h, PLBM_ERR_ARG, "null lattice handle");
-    for (int buf : {a, b})
-        PLBM_REQUIRE(buf >= 0 && buf < h->nf, PLBM_ERR_ARG,
-                     "buffer id " + std::to_string(buf) + " out of range [0," +
-                         std::to_string(h->nf) + ")");
+    PLBM_REQUIRE(buf >= 0 && buf < h->nf, PLBM_ERR_ARG,
+                 "buffer id " + std::to_string(buf) + " out of range [0," +
+                     std::to_string(h->nf) + ")");
+    return PLBM_OK;
+}
+
+// The same in entry points that a graph can hold: one slot, or a and b.
+static int use_buf(plbm_lattice *h, int a, int b = 0) {
+    PLBM_TRY(check_buf(h, a));
+    PLBM_TRY(check_buf(h, b));
     note_capture(h);
     return PLBM_OK;
 }
@@ -816,7 +821,7 @@ int plbm_download_f(plbm_lattice *h, int buf, double *f, int ld) try {
 
 int plbm_equilibrium_init_dev(plbm_lattice *h, int buf, const double *rho, const double *ux,
                               const double *uy) try {
-    PLBM_TRY(check_buf(h, buf));
+    PLBM_TRY(use_buf(h, buf));
     PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
     return dispatch_storage(h->storage, [&](auto S) {
         hipLaunchKernelGGL(k_equilibrium<decltype(S)::value>, cell_grid(h), dim3(256), 0,
@@ -846,7 +851,7 @@ int plbm_equilibrium_init(plbm_lattice *h, int buf, const double *rho, const dou
 }
 
 int plbm_step(plbm_lattice *h, int model, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src, dst));
+    PLBM_TRY(use_buf(h, src, dst));
     PLBM_REQUIRE(src != dst, PLBM_ERR_ARG, "fused step needs distinct src and dst buffers");
     PLBM_TRY(require_params(h));
     return launch_step(h, model, h->f[src], h->f[dst]);
@@ -859,7 +864,7 @@ int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) try {
     PLBM_REQUIRE(nsteps >= 0, PLBM_ERR_ARG, "nsteps must be >= 0");
     PLBM_REQUIRE(model >= PLBM_BGK && model <= PLBM_BGK_SPLIT, PLBM_ERR_ARG,
                  "unknown collision model " + std::to_string(model));
-    PLBM_TRY(check_buf(h, *iold, *inew));
+    PLBM_TRY(use_buf(h, *iold, *inew));
     PLBM_REQUIRE(*iold != *inew, PLBM_ERR_ARG, "iold == inew");
     PLBM_TRY(require_params(h));
     return run_steps(h, model, nsteps, iold, inew);
@@ -868,7 +873,7 @@ int plbm_run(plbm_lattice *h, int model, int nsteps, int *iold, int *inew) try {
 }
 
 int plbm_stream(plbm_lattice *h, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src, dst));
+    PLBM_TRY(use_buf(h, src, dst));
     PLBM_REQUIRE(src != dst, PLBM_ERR_ARG, "streaming needs distinct src and dst buffers");
     return dispatch_storage(h->storage, [&](auto S) {
         using T = typename Traits<decltype(S)::value>::T;
@@ -883,7 +888,7 @@ int plbm_stream(plbm_lattice *h, int src, int dst) try {
 }
 
 int plbm_collide(plbm_lattice *h, int model, int buf) try {
-    PLBM_TRY(check_buf(h, buf));
+    PLBM_TRY(use_buf(h, buf));
     PLBM_TRY(require_params(h));
     StepArgs a = make_args(h, h->f[buf], h->f[buf]);
     PLBM_REQUIRE(model >= PLBM_BGK && model <= PLBM_BGK_SPLIT, PLBM_ERR_ARG,
@@ -901,7 +906,7 @@ int plbm_collide(plbm_lattice *h, int model, int buf) try {
 }
 
 int plbm_copy(plbm_lattice *h, int src, int dst) try {
-    PLBM_TRY(check_buf(h, src, dst));
+    PLBM_TRY(use_buf(h, src, dst));
     if (src == dst) return PLBM_OK;
     PLBM_HIP(hipMemcpyAsync(h->f[dst], h->f[src], h->elems * storage_bytes(h->storage),
                             hipMemcpyDeviceToDevice, h->stream));
@@ -924,7 +929,7 @@ static int launch_macros(plbm_lattice *h, int buf, size_t x0, size_t cols, doubl
 }
 
 int plbm_macros_dev(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) try {
-    PLBM_TRY(check_buf(h, buf));
+    PLBM_TRY(use_buf(h, buf));
     PLBM_REQUIRE(rho && ux && uy, PLBM_ERR_ARG, "null field pointer");
     return launch_macros(h, buf, 0, (size_t)h->nx, rho, ux, uy);
 } catch (...) {
@@ -955,7 +960,7 @@ int plbm_macros(plbm_lattice *h, int buf, double *rho, double *ux, double *uy) t
 
 int plbm_reduce_dev(plbm_lattice *h, int buf, const double *uxa, const double *uya,
                     double out[PLBM_NRED]) try {
-    PLBM_TRY(check_buf(h, buf));
+    PLBM_TRY(use_buf(h, buf));
     PLBM_REQUIRE(out, PLBM_ERR_ARG, "null output");
     PLBM_REQUIRE((uxa == nullptr) == (uya == nullptr), PLBM_ERR_ARG,
                  "uxa and uya must both be given or both be NULL");
@@ -971,7 +976,7 @@ int plbm_reduce_dev(plbm_lattice *h, int buf, const double *uxa, const double *u
 
 int plbm_reduce_static(plbm_lattice *h, int buf, const double *uxa, const double *uya,
                        double *out_dev) try {
-    PLBM_TRY(check_buf(h, buf));
+    PLBM_TRY(use_buf(h, buf));
     PLBM_REQUIRE(out_dev, PLBM_ERR_ARG, "null output");
     PLBM_REQUIRE((uxa == nullptr) == (uya == nullptr), PLBM_ERR_ARG,
                  "uxa and uya must both be given or both be NULL");
