@@ -354,15 +354,14 @@ def config2_leg(P, torch, stream, steps=2000):
 
 
 def schemes_leg(P, torch, args, stream, fields):
-    """The other schemes on the same 8192^2 FP64 start: DUGKS (src/periodic_dugks.F90) as
-    the fused two-kernel step and as the reference's collide + stream sequence, and the
+    """The other schemes on the same 8192^2 FP64 start: DUGKS (src/periodic_dugks.F90)
+    through plbm_dugks_step and as the reference's collide + stream sequence, and the
     finite-volume / finite-difference streaming operators (src/fvm_bardow.F90:393-893)
     with collide_bgk as perform_step runs them (one fused pass per step), and the same
-    pair through plbm_run_op (temporally blocked passes).  Algorithmic bytes per cell and
-    step: fused DUGKS 360 (collide: read 72 + write 72; flux: read ft 72 + f 72, write
-    72), reference-form DUGKS 432, stream operator + BGK 144; a temporally blocked pass
-    moves 144 per cell for all of its steps, and the pass forms report the bytes per
-    cell and step averaged over the timed run."""
+    pair through plbm_run_op.  Algorithmic bytes per cell and step: reference-form DUGKS
+    432, stream operator + BGK 144; a temporally blocked pass moves 144 per cell for all of
+    its steps, the last of a run 216, and the pass forms report the bytes per cell and step
+    averaged over the timed run."""
     n = args.n
     cells = n * n
     tau = 3.0 * NU
@@ -388,25 +387,23 @@ def schemes_leg(P, torch, args, stream, fields):
                 "bytes_per_cell": round(bpc, 2), "gbs": round(bpc * cells / ms / 1e6, 1),
                 "frac_of_peak": round(bpc * cells / ms / 1e6 / HBM_PEAK_GBS, 4)}
 
-    def run_bytes(nsteps, ns, pass_b, single_b, last_b):
-        """Bytes per cell and step of a run that does nsteps - 1 steps in passes of up to
-        ns steps (a remainder of one as a single step) and the last as a single step."""
-        total, done = 0, 0
-        while done < nsteps - 1:
-            k = min(ns, nsteps - 1 - done)
-            total += single_b if k == 1 else pass_b
-            done += k
-        return (total + last_b) / nsteps
+    def run_bytes(nsteps, depth):
+        """Bytes per cell and step of a run in column walks of up to `depth` steps: 144 a
+        pass, and 72 more for the last, which also stores what the other slot holds."""
+        passes = 1 + -(-(nsteps - min(depth, nsteps)) // depth)
+        return (144 * passes + 72) / nsteps
+
+    # the automatic depths of the walks, which grids of more than 10^6 cells take (the getters
+    # report what can be set: at most 3)
+    dugks_depth, op_depth = 3, 4
 
     steps = args.next_steps
     out = {"grid": [n, n], "storage": "f64", "steps": steps}
     ms = timed(lambda k: lat.dugks_step(0, 1, k, 1.0, om_full, om_half), steps, 4)
-    dns = lat.dugks_get_steps_per_pass()
-    out["dugks_fused"] = rec(ms, run_bytes(steps, dns, 144, 360, 360))
-    out["dugks_fused"]["steps_per_pass"] = dns
-    out["dugks_fused"]["note"] = ("all steps but the last in temporally blocked passes "
-                                  "(144 B per cell per pass), the last as collide + flux "
-                                  "(360 B per cell)")
+    out["dugks_fused"] = rec(ms, run_bytes(steps, dugks_depth))
+    out["dugks_fused"]["steps_per_pass"] = dugks_depth
+    out["dugks_fused"]["note"] = ("temporally blocked passes (144 B per cell per pass), the "
+                                  "last also storing the half-collided state (216 B per cell)")
 
     def dugks_ref(k):
         for s in range(k):
@@ -419,11 +416,10 @@ def schemes_leg(P, torch, args, stream, fields):
             for s in range(k):
                 lat.step_op(op, "bgk", s % 2, 1 - s % 2, 1.0)
         out[f"stream_{op}+bgk"] = rec(timed(run, steps, 2), 144)
-        ons = lat.get_op_steps_per_pass(op, "bgk")
         out[f"stream_{op}+bgk_passes"] = rec(
             timed(lambda k, op=op: lat.run_op(op, "bgk", k, 0, 1, 1.0), steps, 4),
-            run_bytes(steps, ons, 144, 144, 144))
-        out[f"stream_{op}+bgk_passes"]["steps_per_pass"] = ons
+            run_bytes(steps, op_depth))
+        out[f"stream_{op}+bgk_passes"]["steps_per_pass"] = op_depth
     lat.close()
     torch.cuda.empty_cache()
     return out
