@@ -167,8 +167,9 @@ int plbm_step_op(plbm_lattice *h, int op, int model, int src, int dst, double dt
  * with the reference's buffer bookkeeping as plbm_run (each step reads *iold, writes
  * *inew, swaps them).  In FP64 storage the steps run in temporally blocked passes of up
  * to plbm_set_op_steps_per_pass steps, the last pass also writing the state one step
- * back into the lattice's third buffer as plbm_run does (bit-identical to single steps;
- * the slots may exchange their device storage, as in plbm_run).  Asynchronous. */
+ * back into the lattice's third buffer as plbm_run does (bit-identical to single steps but
+ * for the sign of zeros, see fd_update in csrc/fd_ops.hpp; the slots may exchange their
+ * device storage, as in plbm_run).  Asynchronous. */
 int plbm_run_op(plbm_lattice *h, int op, int model, int nsteps, int *iold, int *inew,
                 double dt);
 /* Pass depth of plbm_run_op: 1 = single fused steps, 2..3 = passes (FP64 storage only),
@@ -207,8 +208,8 @@ int plbm_dugks_step(plbm_lattice *h, int iold, int inew, int nsteps, double dt,
  * steps but the last in temporally blocked passes of up to this many steps over device
  * memory; 0 (default) = chosen from the grid size, the last pass also storing the
  * half-collided state (plbm_set_pass_lag_buffer; without it, and after a captured call, as
- * 2..3).  Bit-identical for every value.  The getter returns the depth for equal rates as
- * far as it can be set: 3 where the choice is deeper. */
+ * 2..3).  Bit-identical for every value but for the sign of zeros.  The getter returns the
+ * depth for equal rates as far as it can be set: 3 where the choice is deeper. */
 int plbm_dugks_set_steps_per_pass(plbm_lattice *h, int steps);
 /* DUGKS as the reference builds it with -DDUGKS (src/periodic_dugks.F90:68,199,267,308):
  * the stream relaxes the interpolated face values of every face towards the face's own
@@ -280,7 +281,8 @@ double plbm_magic_number(double le, double ld);
 /* ---------------------------------------------------------------- launch shape */
 
 /* Launch shape of the fused step for one model: threads per workgroup (multiple of 64 in
- * [64, 1024]) and XCD-contiguous workgroup renumbering (0/1).  Default 256 / 1. */
+ * [64, 1024]) and XCD-contiguous workgroup renumbering (0/1).  Default 1, and 256 threads, or
+ * 128 on columns of up to 1024 cells that 256 would pad by more. */
 int plbm_set_launch(plbm_lattice *h, int model, int block, int xcd_remap);
 int plbm_get_launch(const plbm_lattice *h, int model, int *block, int *xcd_remap);
 /* Temporal blocking of plbm_run: steps advanced per pass over HBM (1 = the single-step
@@ -304,7 +306,8 @@ int plbm_get_steps_per_launch(const plbm_lattice *h, int model, int *steps);
  * 56 (F64 / F64S) or 48 (F32S / F16S) rows is cut into `segments` column ranges of nearly
  * equal length, one wavefront each (a grid small enough for tiles then walks columns too);
  * 0 = chosen from the grid (as many as fill the chip best, each of at least 8 columns).
- * Results do not depend on it in F64 storage; the others agree to roundoff.  The get variant reports the setting. */
+ * Results do not depend on it in F64 storage; the others agree to roundoff.  The get variant
+ * reports the setting. */
 int plbm_set_pass_segments(plbm_lattice *h, int segments);
 int plbm_get_pass_segments(const plbm_lattice *h, int *segments);
 /* Third population buffer of plbm_run / plbm_run_op in passes (engine extension, no
@@ -398,8 +401,9 @@ int plbm_batch_autotune(plbm_batch *b, int steps, double *best_ms);
  * States are checkpointed every checkpoint_every steps; the reverse sweep recomputes each
  * segment but the last, whose states the forward call keeps, and runs the reverse steps in
  * passes of several as well.  storage: PLBM_F64, PLBM_F64S or PLBM_F32S (FP32
- * forward steps and checkpoints); the adjoint state is FP64 for every storage.  All field pointers are device pointers to (ny, nx) Fortran-order
- * FP64 arrays; the initial fields must stay valid until the backward call. */
+ * forward steps and checkpoints); the adjoint state is FP64 for every storage.  All field
+ * pointers are device pointers to (ny, nx) Fortran-order FP64 arrays; the initial fields must
+ * stay valid until the last backward call. */
 typedef struct plbm_adjoint plbm_adjoint;
 int plbm_adjoint_create(int nx, int ny, int storage, int nsteps, int checkpoint_every,
                         plbm_adjoint **out);
